@@ -6,6 +6,7 @@
 // MXCSR (colizig_cuda.cu:22-29): the GPU runtime must not leak FTZ/DAZ into
 // the engine's CPU float math.
 #include "cz_grouped.h"
+#include "cz_native.h"
 #include "cz_fused.h"
 #include "cz_lru.h"
 #include "cz_sched.h"
@@ -451,8 +452,38 @@ bool rms_rows_write_sgate(const StepArgs &A) {
 
 // y[S][O] = x[S][I] . W^T for NativeMatrix rows (f32: dotF32; BF16: dotBf16,
 // tensors.zig:114-119), bit for bit.
+template <int TG, int TH>
+void launch_native_mfma_t(float *y, const float *x, const uint16_t *w, int S, int I, int O, hipStream_t st) {
+    constexpr int T = 4 * TG * TH, R = 128 / TH;  // tokens and rows of a workgroup
+    k_native_mfma<TG, TH><<<dim3(std::min((O + R - 1) / R, 256), (S + T - 1) / T), 512, (size_t)T * I * sizeof(float),
+                            st>>>(y, x, w, (uint32_t)S, (uint32_t)I, (uint32_t)O);
+}
+
+// BF16 rows on several tokens through the f32 matrix cores (k_native_mfma).  A
+// wave takes a whole 16-row tile, about 20 us at 2048 columns and 35-40 at 4096
+// however few tiles there are, so the row kernel (two rows a wave) keeps the
+// small products: 16384 x 2048 at 8 tokens 34 against 25 us, 8192 x 2048 at 8
+// 17 / 25, 4096 x 2048 at 64 67 / 27; 8192 x 4096 at 8 40 / 42, 2048 x 4096 at
+// 64 106 / 41.  The tokens, in groups of four, are spread evenly over passes
+// that fit LDS (128 KiB).
+constexpr int64_t kNativeMfmaDots = 3 << 15;
+bool launch_native_mfma(float *y, const float *x, const uint16_t *w, int S, int I, int O, hipStream_t st) {
+    if (S < 2 || S > 4 * 65535 || I % 256 || I > 8192 || (int64_t)S * O < kNativeMfmaDots) return false;
+    const int fit = std::min(4, (128 << 10) / (16 * I)), groups = (S + 3) / 4;  // fit >= 1
+    const int passes = (groups + fit - 1) / fit;
+    switch ((groups + passes - 1) / passes) {  // token groups of a pass, evenly
+        case 1: launch_native_mfma_t<1, 1>(y, x, w, S, I, O, st); break;
+        case 2: launch_native_mfma_t<2, 1>(y, x, w, S, I, O, st); break;
+        case 3: launch_native_mfma_t<3, 1>(y, x, w, S, I, O, st); break;
+        default: launch_native_mfma_t<2, 2>(y, x, w, S, I, O, st); break;
+    }
+    return true;
+}
+
 template <typename T>
 void launch_gemv_native(float *y, const float *x, const T *w, int S, int I, int O, hipStream_t st) {
+    if constexpr (std::is_same<T, uint16_t>::value)
+        if (launch_native_mfma(y, x, w, S, I, O, st)) return;
     constexpr int WPB = 8;
     const dim3 grid((O + 2 * WPB - 1) / (2 * WPB)), blk(64 * WPB);
     switch ((I % 32) ? 0 : I / 32) {
