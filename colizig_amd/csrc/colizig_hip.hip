@@ -6,6 +6,7 @@
 // MXCSR (colizig_cuda.cu:22-29): the GPU runtime must not leak FTZ/DAZ into
 // the engine's CPU float math.
 #include "cz_grouped.h"
+#include "cz_gemm.h"
 #include "cz_native.h"
 #include "cz_fused.h"
 #include "cz_lru.h"
@@ -1475,11 +1476,52 @@ void launch_gemv_fp8(float *y, const float *x, const uint8_t *w, const float *s,
         k_gemv_fp8<NB, ST, 1><<<(O + 3) / 4, 256, 0, st>>>(y, x, w, s, (uint32_t)S, (uint32_t)O);
 }
 
+template <int MR, int WN, int KS>
+void launch_gemm_f32x_t(GemvMulti G, const float *x, int S, int I, hipStream_t st) {
+    uint32_t ct = 0;
+    for (uint32_t m = 0; m < G.n; ++m) {
+        G.blk0[m] = ct;
+        ct += (G.O[m] + 64 * WN - 1) / (64 * WN);
+    }
+    G.blk0[G.n] = ct;
+    const uint32_t items = ct * (uint32_t)((S + MR - 1) / MR);
+    k_gemm_f32x<MR, WN, KS><<<(items + 7) / 8 * 8, 64 * WN * KS, 0, st>>>(G, x, (uint32_t)S, (uint32_t)I);
+}
+
+// Many-token products on the f16 matrix cores (k_gemm_f32x).  The rule looks at
+// S and I alone, so that a matrix has the same bits in any launch.
+//
+// The GEMV's time grows with S, the products' hardly up to 48 tokens (16-row
+// tiles, K over four waves): 2048 columns 11 us against 14 (512 rows) and 21
+// (4096) at 16 tokens, 11 against 11 and 17 at 12; 4096 columns 19 against 23
+// (2048 rows) and 37 (4096) at 8, 512 columns 5.5 against 5.7 at 16.  32-row
+// tiles with K over two wave groups from there (q, k, v and o at 64 tokens 65
+// against 66 us), and with four waves side by side once the row tiles alone
+// fill the chip (1000 tokens 127 against 139 us, 385 tokens 96 against 84).
+constexpr int kGemmF32xShortTokens = 48, kGemmF32xSplitTokens = 512;
+bool launch_gemm_f32x(const GemvMulti &G, const float *x, int S, int I, hipStream_t st) {
+    if (I % CZ_BLOCK || (S < 16 && (int64_t)S * I < 28672)) return false;
+    if (S <= kGemmF32xShortTokens)
+        launch_gemm_f32x_t<16, 1, 4>(G, x, S, I, st);
+    else if (S <= kGemmF32xSplitTokens)
+        launch_gemm_f32x_t<32, 2, 2>(G, x, S, I, st);
+    else
+        launch_gemm_f32x_t<32, 4, 1>(G, x, S, I, st);
+    return true;
+}
+
 // y[S][O] = x[S][I] . dequant(W)^T on device pointers (matmulFp8's
 // contract, fp8.zig:215-257): the row-parallel GEMV for I = 64 x {4, 8, 16,
 // 32, 48, 64} (rows 16-byte aligned), else the generic kernel.
 void launch_matmul_fp8(float *y, const float *x, const uint8_t *w, const float *s, int S, int I, int O,
                        hipStream_t st) {
+    GemvMulti G{};
+    G.n = 1;
+    G.y[0] = y;
+    G.w[0] = w;
+    G.s[0] = s;
+    G.O[0] = (uint32_t)O;
+    if (launch_gemm_f32x(G, x, S, I, st)) return;
     switch ((I % 64) ? 0 : I / 64) {
         case 4: launch_gemv_fp8<4>(y, x, w, s, S, O, st); return;
         case 8: launch_gemv_fp8<8>(y, x, w, s, S, O, st); return;
@@ -1664,7 +1706,9 @@ extern "C" int colizig_hip_matmul_fp8_dev_multi(int n, float *const *y_devs, con
         G.O[m] = (uint32_t)Os[m];
     }
     const hipStream_t st = pick_stream(stream);
-    switch ((I % 64) ? 0 : I / 64) {
+    const bool many = launch_gemm_f32x(G, x_dev, S, I, st);
+    switch (many ? -1 : (I % 64) ? 0 : I / 64) {
+        case -1: break;
         case 4: launch_gemv_fp8_multi<4>(G, x_dev, S, st); break;
         case 8: launch_gemv_fp8_multi<8>(G, x_dev, S, st); break;
         case 16: launch_gemv_fp8_multi<16>(G, x_dev, S, st); break;

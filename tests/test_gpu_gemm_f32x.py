@@ -1,0 +1,118 @@
+"""Many-token FP8 products at f32 accuracy (k_gemm_f32x): against 64-bit sums
+over tile edges, odd rows and columns, wide ranges of magnitude, infinities
+and NaN.
+
+The bound on the relative L2 error: the f16 hi + lo split keeps 2^-24 of each
+element, a K block's 128 exact products are summed in f32 (at most 24 rounded
+additions, random signs: about sqrt(24) 2^-25), then one FMA per K block:
+about 2e-7 in all; 6e-7 is asserted."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from colizig_amd import _lib, moe, synth
+from tests.helpers import f32_bits, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 6e-7
+
+
+def _dequant(w, s):
+    import torch
+
+    O, I = w.shape
+    f = torch.from_numpy(w).view(torch.float8_e4m3fn).double().numpy()
+    sc = np.repeat(np.repeat(s.astype(np.float64), 128, 0), 128, 1)[:O, :I]
+    return f * sc
+
+
+def _run(xs, mats, I):
+    """Each matrix alone and all in one launch: the same bits."""
+    S = xs.shape[0]
+    hip = _lib.hip()
+    xb = moe.DeviceBuffer(xs.nbytes)
+    xb.upload(xs)
+    yb = [moe.DeviceBuffer((S * w.shape[0] + 32) * 4) for w, _, _ in mats]
+    outs = []
+    try:
+        for b, (w, s, key) in zip(yb, mats):
+            n = S * w.shape[0]
+            b.upload(np.full(n + 32, 7.0, np.float32))
+            moe.matmul_fp8_dev(b.ptr, xb.ptr, S, I, w.shape[0], key)
+            assert hip.colizig_hip_sync() == 0
+            y = b.download(np.empty(n + 32, np.float32))
+            assert (y[n:] == 7.0).all()
+            outs.append(y[:n].reshape(S, -1).copy())
+        moe.matmul_fp8_dev_multi([b.ptr for b in yb], xb.ptr, S, I, [w.shape[0] for w, _, _ in mats],
+                                 [k for _, _, k in mats])
+        assert hip.colizig_hip_sync() == 0
+        for b, o in zip(yb, outs):
+            y = b.download(np.empty(o.size + 32, np.float32))[:o.size].reshape(o.shape)
+            assert np.array_equal(f32_bits(y), f32_bits(o))
+    finally:
+        xb.free()
+        for b in yb:
+            b.free()
+    return outs
+
+
+@pytest.mark.parametrize("S,I,Os", [(16, 2048, (4096, 512, 512)), (31, 128, (130, 7)), (33, 384, (300,)),
+                                    (64, 896, (65, 256, 1)), (385, 512, (4097, 2048)), (97, 4096, (2048,)),
+                                    (1, 2048, (512,)), (12, 2048, (512,)), (200, 768, (2048,)), (513, 512, (300, 64))])
+def test_many_tokens_f32_accuracy(gpu, S, I, Os):
+    print(f"f32x S={S} I={I} O={Os}", flush=True)
+    rng = np.random.default_rng(S * 7 + I)
+    moe.set_vram_budget(1 << 30)
+    try:
+        x = rng.normal(size=(S, I)).astype(np.float32)
+        x *= (10.0 ** rng.integers(-12, 12, size=(S, 1))).astype(np.float32)  # rows far apart
+        x[:, 5] *= 1e-4  # small beside large in one K block
+        mats = []
+        for m, O in enumerate(Os):
+            w, s = synth.block_quantize(rng.normal(0, 0.02, size=(O, I)).astype(np.float32))
+            key = moe.Fp8Matrix.expert_key(60 + m, (S + I + O) % 509, 1)
+            moe.matrix_load(key, w, s)
+            mats.append((w, s, key))
+        for (w, s, _), y in zip(mats, _run(x, mats, I)):
+            x64, wd = x.astype(np.float64), _dequant(w, s)
+            # against the terms' own size, so that a sum that cancels is not held to its small rest
+            err = np.linalg.norm(y - x64 @ wd.T, axis=1) / np.sqrt(((x64 ** 2) @ (wd ** 2).T).sum(1))
+            print(f"  {w.shape}: worst row {err.max():.2e}", flush=True)
+            assert np.sqrt((err ** 2).mean()) < RTOL
+    finally:
+        moe.set_vram_budget(0)
+
+
+@pytest.mark.parametrize("S", [16, 40])
+def test_extreme_values(gpu, S):
+    """Infinities, NaN, zero rows, the largest and smallest floats, a NaN
+    weight and a zero scale: what f32 sums of the same products give."""
+    rng = np.random.default_rng(S)
+    I, O = 256, 96
+    moe.set_vram_budget(1 << 30)
+    try:
+        w, s = synth.block_quantize(np.abs(rng.normal(0, 0.02, size=(O, I))).astype(np.float32) + 0.01)
+        w[3, 200] = 0x7F  # NaN
+        x = np.abs(rng.normal(size=(S, I))).astype(np.float32)
+        x[0, 7] = np.inf
+        x[1, 7] = -np.inf
+        x[2, 9], x[2, 140] = np.inf, -np.inf
+        x[3, 9] = np.nan
+        x[4] = 0.0
+        x[5] = 1e-38
+        x[6] = 3e33  # times 448 and summed: still finite before the block scale, as in f32 sums
+        x[7, 3], x[7, 4] = np.inf, 3e33  # a large finite value beside an infinity stays finite
+        key = moe.Fp8Matrix.expert_key(70, S, 1)
+        moe.matrix_load(key, w, s)
+        y = _run(x, [(w, s, key)], I)[0]
+        with np.errstate(all="ignore"):
+            ref = np.stack([(x.astype(np.float64)[t] * _dequant(w, s)).sum(1) for t in range(S)]).astype(np.float32)
+        assert np.array_equal(np.isnan(y), np.isnan(ref))
+        fin = np.isfinite(ref)
+        assert np.array_equal(y[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
+        # all terms of one sign: no cancellation
+        assert (np.abs(y[fin] - ref[fin]) <= 2e-6 * np.abs(ref[fin]) + 1e-44).all()
+    finally:
+        moe.set_vram_budget(0)
