@@ -365,8 +365,11 @@ uint32_t grouped_max_tiles(const colizig_dims &d, int S) {
     return sk / CZ_GG_M + std::min(d.experts, sk) + 1;
 }
 
+bool grouped_f32x(const colizig_dims &d, int S);
+
 int ensure_work_grouped(const colizig_dims &d, int S) {
     Work &w = g.work;
+    const bool x32 = grouped_f32x(d, S);
     const size_t s = (size_t)S, sk = s * d.topk, mt = grouped_max_tiles(d, S);
     if (grow(&w.counts, &w.cap_counts, (size_t)d.experts) || grow(&w.offsets, &w.cap_offsets, (size_t)d.experts + 1) ||
         grow(&w.sorted_slot, &w.cap_sorted, sk) || grow(&w.slot_pos, &w.cap_slot_pos, sk) ||
@@ -375,12 +378,12 @@ int ensure_work_grouped(const colizig_dims &d, int S) {
         grow(&w.o, &w.cap_o, sk * d.hidden) || grow(&w.os, &w.cap_os, std::max<size_t>(1, s * d.hidden)) ||
         // the GEMM operands of the active mode only: f16 hi + lo splits, or
         // three E4M3 terms and their exponents
-        (!g.prefill_fp8 &&
+        (!x32 && !g.prefill_fp8 &&
          (grow(&w.xh, &w.cap_xh, s * d.hidden) || grow(&w.xl, &w.cap_xl, s * d.hidden) ||
           grow(&w.hh, &w.cap_hh, sk * d.inter) || grow(&w.hl, &w.cap_hl, sk * d.inter) ||
           grow(&w.hsh, &w.cap_hsh, std::max<size_t>(1, s * d.shared_inter)) ||
           grow(&w.hsl, &w.cap_hsl, std::max<size_t>(1, s * d.shared_inter)))) ||
-        (g.prefill_fp8 &&
+        (!x32 && g.prefill_fp8 &&
          (grow(&w.xq, &w.cap_xq, 3 * s * d.hidden) || grow(&w.xe, &w.cap_xe, 3 * s * d.hidden / 32) ||
           grow(&w.hq, &w.cap_hq, 3 * sk * d.inter) || grow(&w.he, &w.cap_he, 3 * sk * d.inter / 32) ||
           grow(&w.hsq, &w.cap_hsq, std::max<size_t>(1, 3 * s * d.shared_inter)) ||
@@ -392,9 +395,20 @@ int ensure_work_grouped(const colizig_dims &d, int S) {
 }
 
 
+// Past CZ_DISPATCH_MAX slots the grouped GEMMs keep f32's accuracy, which such
+// calls have always had (k_gg_f32x; the forms that split the rows beforehand
+// hold 12 or 22 bits), up to kWideMaxSlots: their O rows are 4 H bytes a slot
+// (0.5 GB at 65,536 slots of 2048).  2000 tokens of a Qwen3-30B-A3B layer
+// (16,000 slots): 10,800 us with the per-token kernels, 555 us.
+constexpr size_t kWideMaxSlots = 65536;
+bool grouped_f32x(const colizig_dims &d, int S) {
+    const size_t sk = (size_t)S * d.topk;
+    return sk > CZ_DISPATCH_MAX && sk <= kWideMaxSlots;
+}
+
 bool grouped_ok(const colizig_dims &d, int S) {
     return S >= kGroupedMinTokens && d.hidden % 256 == 0 && d.inter % 128 == 0 && d.shared_inter % 128 == 0 &&
-           (size_t)S * d.topk <= CZ_DISPATCH_MAX;
+           ((size_t)S * d.topk <= CZ_DISPATCH_MAX || grouped_f32x(d, S));
 }
 
 void free_layer(LayerHost &L) {
@@ -774,6 +788,7 @@ StepArgs grouped_args(const LayerHost &Lh, const float *x, int S, float *out, in
                       float *xn_trace, uint32_t *idx_trace, float *gates_trace) {
     StepArgs A = step_args(Lh, x, S, out, rms, eps, xres, xn_trace, idx_trace, gates_trace);
     Work &w = g.work;
+    if (grouped_f32x(Lh.d, S)) return A;  // k_gg_f32x reads f32 rows
     if (rms && !g.prefill_fp8) {
         A.xh = w.xh;
         A.xl = w.xl;
@@ -808,7 +823,7 @@ int launch_grouped(const LayerHost &Lh, const float *x, int S, float *out, int r
     A.rms_ready = rms_ready ? 1u : 0u;
     const LayerDev &L = A.L;
     Work &w = g.work;
-    const bool f8 = g.prefill_fp8;
+    const bool x32 = grouped_f32x(Lh.d, S), f8 = g.prefill_fp8 && !x32;
     const bool xq_rms = A.xq != nullptr;
     launch_router(A, st);
     if (Lh.shn_dtype >= 0) {
@@ -835,8 +850,8 @@ int launch_grouped(const LayerHost &Lh, const float *x, int S, float *out, int r
     G.tile_row0 = w.tile_row0;
     G.ntiles = w.ntiles;
     G.max_tiles = grouped_max_tiles(Lh.d, S);
-    G.xh = rms || f8 ? nullptr : w.xh;  // no RMS rows kernel: the routing kernel splits x
-    G.xl = rms || f8 ? nullptr : w.xl;
+    G.xh = rms || f8 || x32 ? nullptr : w.xh;  // no RMS rows kernel: the routing kernel splits x
+    G.xl = rms || f8 || x32 ? nullptr : w.xl;
     G.hh = w.hh;
     G.hl = w.hl;
     G.hsh = w.hsh;
@@ -853,7 +868,10 @@ int launch_grouped(const LayerHost &Lh, const float *x, int S, float *out, int r
         default: launch_route_tokens<16>(G, st); break;
     }
     G.usage = L.usage;
-    k_dispatch<<<1, 1024, 0, st>>>(G);
+    if (x32)
+        k_dispatch<true><<<1, 1024, 0, st>>>(G);
+    else
+        k_dispatch<false><<<1, 1024, 0, st>>>(G);
     const uint32_t mts = (uint32_t)(S + CZ_GG_M - 1) / CZ_GG_M;
     const uint64_t sk = (uint64_t)S * L.K;
     auto quant3 = [&](const float *src, uint64_t rows, uint32_t K, uint8_t *q, uint8_t *e) {
@@ -909,7 +927,11 @@ int launch_grouped(const LayerHost &Lh, const float *x, int S, float *out, int r
         Q.rows_total = (uint32_t)S;
     }
     const uint32_t qu = L.SI ? (mts * (L.SI / cu) + 7) / 8 * 8 : 0u;
-    if (f8)
+    if (x32) {
+        P.c = w.h;
+        Q.c = w.hs;
+        k_gg_f32x<GG_GATEUP><<<qu + gg_blocks(G.max_tiles, L.I, cu), 256, 0, st>>>(G, P, Q, G.xn, G.xn);
+    } else if (f8)
         k_gg8<GG_GATEUP><<<qu + gg_blocks(G.max_tiles, L.I, cu), 256, 0, st>>>(G, P, Q);
     else
         k_gg<GG_GATEUP><<<qu + gg_blocks(G.max_tiles, L.I, cu), 256, 0, st>>>(G, P, Q);
@@ -951,7 +973,9 @@ int launch_grouped(const LayerHost &Lh, const float *x, int S, float *out, int r
         QD.ae_plane = (uint64_t)S * L.SI / 32;
     }
     const uint32_t qd = L.SI ? (mts * (L.H / cd) + 7) / 8 * 8 : 0u;
-    if (f8)
+    if (x32) {
+        k_gg_f32x<GG_DOWN><<<qd + gg_blocks(G.max_tiles, L.H, cd), 256, 0, st>>>(G, D, QD, w.h, w.hs);
+    } else if (f8)
         k_gg8<GG_DOWN><<<qd + gg_blocks(G.max_tiles, L.H, cd), 256, 0, st>>>(G, D, QD);
     else
         k_gg<GG_DOWN><<<qd + gg_blocks(G.max_tiles, L.H, cd), 256, 0, st>>>(G, D, QD);

@@ -170,8 +170,10 @@ __global__ __launch_bounds__(256) void k_route_tokens(GroupArgs G) {
 
 // ---------------------------------------------------------------------------
 // dispatch (moe.zig:597-612: the routed rows grouped by expert): one
-// workgroup of 1024 threads (16 waves) over the S*K slot ids (S*K <=
-// CZ_DISPATCH_MAX, E <= CZ_MAX_E).  Each slot takes its rank among its
+// workgroup of 1024 threads (16 waves) over the S*K slot ids (E <= CZ_MAX_E).
+// Up to CZ_DISPATCH_MAX slots a thread holds its slots' experts and ranks in
+// registers; above (WIDE) it passes over them in that many at a time, the ranks
+// waiting in slot_pos (16,000 slots: 17-23 us).  Each slot takes its rank among its
 // expert's rows from an LDS atomic on the expert's count, the offsets come
 // from one prefix of the counts, and the slot goes to offset + rank.  Rows of
 // one expert come in the order the atomics were served, which is not fixed;
@@ -180,6 +182,7 @@ __global__ __launch_bounds__(256) void k_route_tokens(GroupArgs G) {
 // ---------------------------------------------------------------------------
 #define CZ_DISPATCH_MAX 8192
 
+template <bool WIDE>
 __global__ __launch_bounds__(1024) void k_dispatch(GroupArgs G) {
     const LayerDev &L = G.L;
     const uint32_t E = L.E, SK = (uint32_t)G.S * L.K;
@@ -187,19 +190,30 @@ __global__ __launch_bounds__(1024) void k_dispatch(GroupArgs G) {
     __shared__ uint32_t s_cnt[CZ_MAX_E];
     __shared__ uint32_t s_off[CZ_MAX_E + 1];
     const uint32_t tid = threadIdx.x, lane = cz_lane();
+    uint32_t ev[NQ], rk[NQ];
     // the slots' expert ids: all of a thread's loads in flight at once
     // (indices past SK re-read slot SK - 1, unconditionally, so the loads are
     // not serialised by branches)
-    uint32_t ev[NQ], rk[NQ];
+    auto ids = [&](uint32_t b) {
 #pragma unroll
-    for (uint32_t q = 0; q < NQ; ++q) ev[q] = G.idx[min(tid + 1024u * q, SK - 1)];
+        for (uint32_t q = 0; q < NQ; ++q) ev[q] = G.idx[min(b + tid + 1024u * q, SK - 1)];
 #pragma unroll
-    for (uint32_t q = 0; q < NQ; ++q) ev[q] = min(ev[q], E - 1);
+        for (uint32_t q = 0; q < NQ; ++q) ev[q] = min(ev[q], E - 1);
+    };
+    ids(0);
     for (uint32_t i = tid; i < E; i += blockDim.x) s_cnt[i] = 0;
     __syncthreads();
+    for (uint32_t b = 0; b < (WIDE ? SK : 1u); b += CZ_DISPATCH_MAX) {
+        if (WIDE && b) ids(b);
 #pragma unroll
-    for (uint32_t q = 0; q < NQ; ++q)
-        if (tid + 1024u * q < SK) rk[q] = atomicAdd(&s_cnt[ev[q]], 1u);
+        for (uint32_t q = 0; q < NQ; ++q) {
+            const uint32_t i = b + tid + 1024u * q;
+            if (i < SK) {
+                rk[q] = atomicAdd(&s_cnt[ev[q]], 1u);
+                if (WIDE) G.slot_pos[i] = rk[q];  // kept there until the offsets are known
+            }
+        }
+    }
     __syncthreads();
     if (tid < 64) {  // one wave: exclusive prefix of counts and of M-tile counts
         uint32_t acc = 0, tacc = 0;
@@ -235,13 +249,20 @@ __global__ __launch_bounds__(1024) void k_dispatch(GroupArgs G) {
             if (G.usage && s_cnt[e]) atomicAdd(G.usage + e, (unsigned long long)s_cnt[e]);
         }
     }
+    for (uint32_t b = 0; b < (WIDE ? SK : 1u); b += CZ_DISPATCH_MAX) {
+        if (WIDE) {  // the ranks each thread stored itself
+            ids(b);
 #pragma unroll
-    for (uint32_t q = 0; q < NQ; ++q) {
-        const uint32_t i = tid + 1024u * q;
-        if (i < SK) {
-            const uint32_t pos = s_off[ev[q]] + rk[q];
-            G.sorted_slot[pos] = i;
-            G.slot_pos[i] = pos;
+            for (uint32_t q = 0; q < NQ; ++q) rk[q] = G.slot_pos[min(b + tid + 1024u * q, SK - 1)];
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < NQ; ++q) {
+            const uint32_t i = b + tid + 1024u * q;
+            if (i < SK) {
+                const uint32_t pos = s_off[ev[q]] + rk[q];
+                G.sorted_slot[pos] = i;
+                G.slot_pos[i] = pos;
+            }
         }
     }
 }

@@ -27,7 +27,8 @@ inline uint64_t plan_nblk(uint64_t x) { return (x + 127) / 128; }
 // The forward's scratch for S tokens, byte for byte what the library's
 // decode scratch and, in the grouped regime, its grouped scratch allocate in
 // the given prefill mode (FP8: three E4M3 terms and their exponents of the
-// GEMM operands; f16: hi + lo splits).
+// GEMM operands; f16: hi + lo splits).  Past 8192 slots the products read f32
+// rows and the operands' share is not allocated: an upper bound there.
 inline uint64_t work_bytes(const colizig_dims &d, uint64_t S, bool prefill_fp8) {
     const uint64_t sk = S * d.topk, H = d.hidden, SI = d.shared_inter;
     const uint64_t mt = sk / kPlanTileRows + std::min<uint64_t>(d.experts, sk) + 1;

@@ -1,6 +1,6 @@
-"""Many-token FP8 products at f32 accuracy (k_gemm_f32x): against 64-bit sums
-over tile edges, odd rows and columns, wide ranges of magnitude, infinities
-and NaN.
+"""Many-token FP8 products at f32 accuracy (k_gemm_f32x, k_gg_f32x): against
+64-bit sums over tile edges, odd rows and columns, wide ranges of magnitude,
+infinities and NaN; and layers past 8192 slots against the oracle.
 
 The bound on the relative L2 error: the f16 hi + lo split keeps 2^-24 of each
 element, a K block's 128 exact products are summed in f32 (at most 24 rounded
@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from colizig_amd import _lib, moe, synth
+from oracle import oracle as orc
 from tests.helpers import f32_bits, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -116,3 +117,23 @@ def test_extreme_values(gpu, S):
         assert (np.abs(y[fin] - ref[fin]) <= 2e-6 * np.abs(ref[fin]) + 1e-44).all()
     finally:
         moe.set_vram_budget(0)
+
+
+@pytest.mark.parametrize("H,E,K,I,SI,S", [(256, 16, 8, 128, 0, 1025), (512, 24, 10, 256, 0, 900),
+                                          (256, 64, 16, 384, 256, 600)])
+def test_layer_past_8192_slots(gpu, H, E, K, I, SI, S):
+    print(f"layer H={H} E={E} K={K} I={I} SI={SI} S={S}", flush=True)
+    host = synth.make_layer(H, E, K, I, SI, True, seed=S)
+    L = moe.register_layer(0, host)
+    x = synth.hidden_states(S, H, seed=S)
+    assert _lib.hip().colizig_hip_usage_reset() == 0
+    out, idx, gates = L.forward(x)
+    ro, ri, rg = orc.OracleLayer(host).forward(x)
+    assert np.array_equal(idx, ri)
+    assert np.array_equal(f32_bits(gates), f32_bits(rg))
+    err = rel_l2(out, ro)
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err < 1.5e-6  # three such products, silu, the oracle's own f32 sums
+    counts = np.zeros((1, E), np.uint64)
+    assert _lib.hip().colizig_hip_usage_read(0, 1, E, counts.ctypes.data) == 0
+    assert np.array_equal(counts[0], np.bincount(ri.ravel(), minlength=E).astype(np.uint64))
