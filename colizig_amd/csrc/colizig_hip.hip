@@ -411,6 +411,28 @@ bool grouped_ok(const colizig_dims &d, int S) {
            ((size_t)S * d.topk <= CZ_DISPATCH_MAX || grouped_f32x(d, S));
 }
 
+// Whether a layer call runs the grouped regime.  Past CZ_DISPATCH_MAX slots
+// only with its scratch there: without room for the O rows such calls keep the
+// per-token kernels, whose scratch is smaller.
+bool use_grouped(const colizig_dims &d, int S) {
+    if (!grouped_ok(d, S)) return false;
+    if (!grouped_f32x(d, S)) return true;
+    const Work &w = g.work;
+    const size_t s = (size_t)S, sk = s * d.topk, mt = grouped_max_tiles(d, S);
+    return w.cap_counts >= d.experts && w.cap_offsets > d.experts && w.cap_sorted >= sk && w.cap_slot_pos >= sk &&
+           w.cap_tok_order >= sk && w.cap_tiles >= mt && w.cap_tiles2 >= mt && w.cap_ntiles >= 1 &&
+           w.cap_o >= sk * d.hidden && w.cap_os >= s * d.hidden;
+}
+
+// The grouped regime's scratch, where a call of S tokens takes it.
+int ensure_grouped(const colizig_dims &d, int S) {
+    if (!grouped_ok(d, S)) return 0;
+    const int rc = ensure_work_grouped(d, S);
+    if (rc == 0 || !grouped_f32x(d, S)) return rc;
+    (void)hipGetLastError();  // the failed allocation is no launch's error
+    return 0;
+}
+
 void free_layer(LayerHost &L) {
     if (!L.streamed())
         for (void *p : {(void *)L.ew, (void *)L.es})
@@ -809,7 +831,7 @@ StepArgs grouped_args(const LayerHost &Lh, const float *x, int S, float *out, in
 constexpr int kCombineRmsMinTokens = 256;
 bool combine_rms_ok(const LayerHost &Lh, const LayerHost &Ln, int S) {
     const uint32_t q = (Lh.d.hidden / 4 + 255) / 256;
-    return S >= kCombineRmsMinTokens && grouped_ok(Lh.d, S) && grouped_ok(Ln.d, S) && Ln.d.hidden == Lh.d.hidden &&
+    return S >= kCombineRmsMinTokens && use_grouped(Lh.d, S) && use_grouped(Ln.d, S) && Ln.d.hidden == Lh.d.hidden &&
            !Ln.router_bf16 &&
            Lh.shn_dtype < 0 && Ln.shn_dtype < 0 && rms_rows_wg(Ln, S) && q >= 1 && q <= 8;
 }
@@ -1177,7 +1199,7 @@ int chain_fused_prepare(uint32_t layer0, uint32_t n, int S) {
 int launch_layer(const LayerHost &Lh, const float *x, int S, float *out, int rms, float eps, const float *xres,
                  float *xn_trace, uint32_t *idx_trace, float *gates_trace, hipStream_t st, bool rms_ready = false,
                  const LayerHost *next = nullptr, float *next_xn_trace = nullptr) {
-    if (grouped_ok(Lh.d, S))
+    if (use_grouped(Lh.d, S))
         return launch_grouped(Lh, x, S, out, rms, eps, xres, xn_trace, idx_trace, gates_trace, st, rms_ready, next,
                               next_xn_trace);
     const StepArgs A = step_args(Lh, x, S, out, rms, eps, xres, xn_trace, idx_trace, gates_trace);
@@ -1987,7 +2009,7 @@ extern "C" int colizig_hip_moe_forward_dev(uint32_t layer, const float *x_dev, i
     int rc = check_layer_ready(L, layer);
     if (rc) return rc;
     if ((rc = ensure_work(L->d, S))) return rc;
-    if (grouped_ok(L->d, S) && (rc = ensure_work_grouped(L->d, S))) return rc;
+    if ((rc = ensure_grouped(L->d, S))) return rc;
     if (L->streamed()) {
         if ((rc = ensure_work_grouped(L->d, S)) || (rc = ensure_h_idx(S))) return rc ? rc : -2;
         rc = run_streamed_layer(*L, layer, x_dev, S, out_dev, 0, 0.0f, nullptr, nullptr, 0, pick_stream(stream),
@@ -2106,7 +2128,7 @@ extern "C" int colizig_hip_moe_forward(uint32_t layer, const float *x, int S, fl
     int rc = check_layer_ready(L, layer);
     if (rc) return rc;
     if ((rc = ensure_work(L->d, S))) return rc;
-    if (grouped_ok(L->d, S) && (rc = ensure_work_grouped(L->d, S))) return rc;
+    if ((rc = ensure_grouped(L->d, S))) return rc;
     const size_t xb = (size_t)S * L->d.hidden * sizeof(float);
     const size_t kb = (size_t)S * L->d.topk * sizeof(float);
     if (ensure_host(xb + 2 * kb)) return -2;
@@ -2143,7 +2165,7 @@ static int chain_enqueue(uint32_t layer0, uint32_t nlayers, float *x_dev, int S,
             return -1;
         }
         if ((rc = ensure_work(L->d, S))) return rc;
-        if (grouped_ok(L->d, S) && (rc = ensure_work_grouped(L->d, S))) return rc;
+        if ((rc = ensure_grouped(L->d, S))) return rc;
     }
     const int fz = chain_fused_prepare(layer0, nlayers, S);
     if (fz < 0) return fz;
@@ -2184,7 +2206,7 @@ extern "C" int64_t colizig_hip_chain_graph_create(uint32_t layer0, uint32_t nlay
         int rc = check_layer_ready(L, layer0 + l);
         if (rc) return rc;
         if ((rc = ensure_work(L->d, S))) return rc;
-        if (grouped_ok(L->d, S) && (rc = ensure_work_grouped(L->d, S))) return rc;
+        if ((rc = ensure_grouped(L->d, S))) return rc;
     }
     if (const int fz = chain_fused_prepare(layer0, nlayers, S); fz < 0) return fz;
     CZ_CHECK(hipStreamSynchronize(g.stream), -4);
@@ -2417,7 +2439,7 @@ extern "C" int colizig_hip_chain_kernel_times(uint32_t layer0, uint32_t nlayers,
         if (rc) return rc;
         if (L->streamed()) return -1;
         if ((rc = ensure_work(L->d, S))) return rc;
-        if (grouped_ok(L->d, S) && (rc = ensure_work_grouped(L->d, S))) return rc;
+        if ((rc = ensure_grouped(L->d, S))) return rc;
     }
     std::vector<StepArgs> args;
     for (uint32_t l = 0; l < nlayers; ++l) {
@@ -2991,7 +3013,7 @@ int run_streamed_layer(LayerHost &L, uint32_t layer, const float *x, int S, floa
         }
         P.last_pred.record(layer, P.h_idx, nk);
     }
-    const bool grouped = grouped_ok(L.d, S);
+    const bool grouped = use_grouped(L.d, S);
     StepArgs A2 = A;  // the decode kernels can take the slots in their arguments
     int rc = stream_resident(L, layer, sel, st, grouped ? nullptr : &A2.L);
     if (rc) return rc;
