@@ -1537,20 +1537,21 @@ void launch_gemm_f32x_t(GemvMulti G, const float *x, int S, int I, hipStream_t s
 // Many-token products on the f16 matrix cores (k_gemm_f32x).  The rule looks at
 // S and I alone, so that a matrix has the same bits in any launch.
 //
-// The GEMV's time grows with S, the products' hardly up to 48 tokens (16-row
+// The GEMV's time grows with S, the products' hardly up to 96 tokens (16-row
 // tiles, K over four waves): 2048 columns 11 us against 14 (512 rows) and 21
 // (4096) at 16 tokens, 11 against 11 and 17 at 12; 4096 columns 19 against 23
-// (2048 rows) and 37 (4096) at 8, 512 columns 5.5 against 5.7 at 16.  32-row
-// tiles with K over two wave groups from there (q, k, v and o at 64 tokens 65
-// against 66 us), and with four waves side by side once the row tiles alone
-// fill the chip (1000 tokens 127 against 139 us, 385 tokens 96 against 84).
-constexpr int kGemmF32xShortTokens = 48, kGemmF32xSplitTokens = 512;
+// (2048 rows) and 37 (4096) at 8, 512 columns 5.5 against 5.7 at 16.  From 129
+// tokens K goes over two wave groups and twice the columns (q, k, v and o: 128
+// tokens 41 against 45 us, 160 tokens 52 against 46, 385 tokens 95 against 71;
+// 32-row tiles 81 there), from 513 four waves stand side by side on 32-row
+// tiles (1000 tokens 127 us, K over two wave groups 139).
+constexpr int kGemmF32xShortTokens = 128, kGemmF32xSplitTokens = 512;
 bool launch_gemm_f32x(const GemvMulti &G, const float *x, int S, int I, hipStream_t st) {
     if (I % CZ_BLOCK || (S < 16 && (int64_t)S * I < 28672)) return false;
     if (S <= kGemmF32xShortTokens)
         launch_gemm_f32x_t<16, 1, 4>(G, x, S, I, st);
     else if (S <= kGemmF32xSplitTokens)
-        launch_gemm_f32x_t<32, 2, 2>(G, x, S, I, st);
+        launch_gemm_f32x_t<16, 2, 2>(G, x, S, I, st);
     else
         launch_gemm_f32x_t<32, 4, 1>(G, x, S, I, st);
     return true;
