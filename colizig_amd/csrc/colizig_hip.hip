@@ -11,6 +11,7 @@
 #include "cz_fused.h"
 #include "cz_lru.h"
 #include "cz_sched.h"
+#include "cz_scratch.h"
 #include "cz_plan.h"
 #include "colizig_hip.h"
 
@@ -326,15 +327,10 @@ int ensure_host(size_t need) {
 
 template <typename T>
 int grow(T **p, size_t *cap, size_t need) {
-    if (*cap >= need) return 0;
-    if (*p) g.retired.push_back((void *)*p);
-    *p = nullptr;
-    *cap = 0;
-    void *q = nullptr;
-    if (hipMalloc(&q, need * sizeof(T)) != hipSuccess) return -1;
-    *p = (T *)q;
-    *cap = need;
-    return 0;
+    return cz::grow_buffer(p, cap, need, g.retired, [](size_t bytes) {
+        void *q = nullptr;
+        return hipMalloc(&q, bytes) == hipSuccess ? q : nullptr;
+    });
 }
 
 // Scratch for S tokens of a layer with dims d (max over callers).

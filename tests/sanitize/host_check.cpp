@@ -11,6 +11,7 @@
 #include <cinttypes>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <random>
 #include <vector>
@@ -18,6 +19,7 @@
 #include "cz_lru.h"
 #include "cz_plan.h"
 #include "cz_sched.h"
+#include "cz_scratch.h"
 
 extern "C" {
 int czgpu_init(const char *lib_path, char *err, size_t errlen);
@@ -198,6 +200,37 @@ static void lru_cases() {
     }
 }
 
+// the forward's scratch when memory runs short: what fitted stays usable
+static void scratch_cases() {
+    size_t left = 1000;  // bytes the stub device has
+    int calls = 0;
+    auto alloc = [&](size_t bytes) -> void * {
+        ++calls;
+        if (bytes > left) return nullptr;
+        left -= bytes;
+        return std::malloc(bytes);
+    };
+    std::vector<void *> retired;
+    float *o = nullptr;
+    size_t cap = 0;
+    // a small layer's buffer, then a large layer's that does not fit: the small
+    // layer's launch (after both, as in a chain) still has its buffer
+    CHECK(cz::grow_buffer(&o, &cap, 100, retired, alloc) == 0 && o && cap == 100);
+    float *const small = o;
+    for (int i = 0; i < 50; ++i) {  // large and small calls in turn: nothing is lost or leaked
+        CHECK(cz::grow_buffer(&o, &cap, 1000, retired, alloc) == -1);
+        CHECK(o == small && cap == 100 && retired.empty());
+        CHECK(cz::grow_buffer(&o, &cap, 100, retired, alloc) == 0 && o == small);
+    }
+    CHECK(left == 600 && calls == 51);
+    // a growth that fits retires the old buffer, once
+    CHECK(cz::grow_buffer(&o, &cap, 150, retired, alloc) == 0 && o != small && cap == 150);
+    CHECK(retired.size() == 1 && retired[0] == small);
+    for (size_t i = 0; i < cap; ++i) o[i] = 1.0f;
+    for (void *q : retired) std::free(q);
+    std::free(o);
+}
+
 static void plan_cases() {
     const uint64_t GB = 1ull << 30;
     const colizig_dims small{512, 16, 4, 256, 0, 1}, q3{2048, 128, 8, 768, 0, 1}, q4{4096, 512, 10, 512, 4096, 1};
@@ -273,6 +306,7 @@ int main(int argc, char **argv) {
     }
     sched_cases();
     predictor_cases();
+    scratch_cases();
     plan_cases();
     lru_cases();
     loader_cases(argv[1], argv[2], argv[3]);
