@@ -325,12 +325,16 @@ int ensure_host(size_t need) {
     return 0;
 }
 
+void *dev_alloc(size_t bytes) {
+    void *q = nullptr;
+    if (hipMalloc(&q, bytes) == hipSuccess) return q;
+    (void)hipGetLastError();  // the caller may go on without: it is no launch's error
+    return nullptr;
+}
+
 template <typename T>
 int grow(T **p, size_t *cap, size_t need) {
-    return cz::grow_buffer(p, cap, need, g.retired, [](size_t bytes) {
-        void *q = nullptr;
-        return hipMalloc(&q, bytes) == hipSuccess ? q : nullptr;
-    });
+    return cz::grow_buffer(p, cap, need, g.retired, dev_alloc);
 }
 
 // Scratch for S tokens of a layer with dims d (max over callers).
@@ -371,7 +375,8 @@ int ensure_work_grouped(const colizig_dims &d, int S) {
         grow(&w.sorted_slot, &w.cap_sorted, sk) || grow(&w.slot_pos, &w.cap_slot_pos, sk) ||
         grow(&w.tok_order, &w.cap_tok_order, sk) || grow(&w.tile_expert, &w.cap_tiles, mt) ||
         grow(&w.tile_row0, &w.cap_tiles2, mt) || grow(&w.ntiles, &w.cap_ntiles, (size_t)1) ||
-        grow(&w.o, &w.cap_o, sk * d.hidden) || grow(&w.os, &w.cap_os, std::max<size_t>(1, s * d.hidden)) ||
+        cz::grow_stepped(&w.o, &w.cap_o, sk * d.hidden, cz::grouped_o_slots(sk) * d.hidden, g.retired, dev_alloc) ||
+        grow(&w.os, &w.cap_os, std::max<size_t>(1, s * d.hidden)) ||
         // the GEMM operands of the active mode only: f16 hi + lo splits, or
         // three E4M3 terms and their exponents
         (!x32 && !g.prefill_fp8 &&
@@ -393,13 +398,12 @@ int ensure_work_grouped(const colizig_dims &d, int S) {
 
 // Past CZ_DISPATCH_MAX slots the grouped GEMMs keep f32's accuracy, which such
 // calls have always had (k_gg_f32x; the forms that split the rows beforehand
-// hold 12 or 22 bits), up to kWideMaxSlots: their O rows are 4 H bytes a slot
+// hold 12 or 22 bits), up to kPlanWideSlots: their O rows are 4 H bytes a slot
 // (0.5 GB at 65,536 slots of 2048).  2000 tokens of a Qwen3-30B-A3B layer
 // (16,000 slots): 10,800 us with the per-token kernels, 555 us.
-constexpr size_t kWideMaxSlots = 65536;
 bool grouped_f32x(const colizig_dims &d, int S) {
     const size_t sk = (size_t)S * d.topk;
-    return sk > CZ_DISPATCH_MAX && sk <= kWideMaxSlots;
+    return sk > CZ_DISPATCH_MAX && sk <= cz::kPlanWideSlots;
 }
 
 bool grouped_ok(const colizig_dims &d, int S) {
@@ -424,9 +428,7 @@ bool use_grouped(const colizig_dims &d, int S) {
 int ensure_grouped(const colizig_dims &d, int S) {
     if (!grouped_ok(d, S)) return 0;
     const int rc = ensure_work_grouped(d, S);
-    if (rc == 0 || !grouped_f32x(d, S)) return rc;
-    (void)hipGetLastError();  // the failed allocation is no launch's error
-    return 0;
+    return grouped_f32x(d, S) ? 0 : rc;
 }
 
 void free_layer(LayerHost &L) {
@@ -3767,7 +3769,8 @@ extern "C" int colizig_hip_predictor_stats(int64_t h, uint64_t *predicted, uint6
 }
 
 // ---- HBM plan (budget.plan, budget.zig:184-264, for one GPU's HBM): cz_plan.h
-static_assert(cz::kPlanTileRows == CZ_GG_M && cz::kPlanGroupedMinTokens == (uint32_t)kGroupedMinTokens,
+static_assert(cz::kPlanDispatchSlots == CZ_DISPATCH_MAX && cz::kPlanTileRows == CZ_GG_M &&
+                  cz::kPlanGroupedMinTokens == (uint32_t)kGroupedMinTokens,
               "the plan's scratch count follows the forward's regimes");
 
 extern "C" int colizig_hip_plan_hbm(const colizig_dims *dims, uint32_t layers, uint64_t hbm_budget,

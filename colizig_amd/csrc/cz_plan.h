@@ -22,13 +22,28 @@ constexpr uint32_t kCapLadder[] = {128, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4};
 constexpr uint32_t kPlanGroupedMinTokens = 16;
 constexpr uint32_t kPlanTileRows = 32;
 
+// Slots (tokens x top-k) up to which the grouped regime keeps its dispatch in
+// one pass, and up to which it runs at all.
+constexpr uint64_t kPlanDispatchSlots = 8192, kPlanWideSlots = 65536;
+
+// O rows the grouped scratch asks for at sk slots.  Past kPlanDispatchSlots they
+// are 4 H bytes a slot, and a growing buffer's predecessors stay until shutdown:
+// powers of two, so that prompts that grow leave less behind than they hold.
+inline uint64_t grouped_o_slots(uint64_t sk) {
+    if (sk <= kPlanDispatchSlots || sk > kPlanWideSlots) return sk;
+    uint64_t n = 2 * kPlanDispatchSlots;
+    while (n < sk) n *= 2;
+    return n;
+}
+
 inline uint64_t plan_nblk(uint64_t x) { return (x + 127) / 128; }
 
 // The forward's scratch for S tokens, byte for byte what the library's
 // decode scratch and, in the grouped regime, its grouped scratch allocate in
 // the given prefill mode (FP8: three E4M3 terms and their exponents of the
 // GEMM operands; f16: hi + lo splits).  Past 8192 slots the products read f32
-// rows and the operands' share is not allocated: an upper bound there.
+// rows, the operands' share is not allocated and the O rows come in steps: an
+// upper bound there.
 inline uint64_t work_bytes(const colizig_dims &d, uint64_t S, bool prefill_fp8) {
     const uint64_t sk = S * d.topk, H = d.hidden, SI = d.shared_inter;
     const uint64_t mt = sk / kPlanTileRows + std::min<uint64_t>(d.experts, sk) + 1;
@@ -36,7 +51,7 @@ inline uint64_t work_bytes(const colizig_dims &d, uint64_t S, bool prefill_fp8) 
     uint64_t b = 4 * (3 * S * H + S * d.experts + 2 * sk + S + sk * d.inter + si);  // xin, out, xn, logits, ..
     if (SI) b += 4 * (2 * S * SI + S * H + S);  // the shared expert's gate, up, down rows and gate
     if (S < kPlanGroupedMinTokens) return b;
-    b += 4 * (2 * (uint64_t)d.experts + 1 + 3 * sk + 2 * mt + 1 + sk * H + std::max<uint64_t>(1, S * H));
+    b += 4 * (2 * (uint64_t)d.experts + 1 + 3 * sk + 2 * mt + 1 + grouped_o_slots(sk) * H + std::max<uint64_t>(1, S * H));
     if (prefill_fp8)
         b += 3 * (S * H + sk * d.inter) + 3 * (S * H + sk * d.inter) / 32 + std::max<uint64_t>(1, 3 * S * SI) +
              std::max<uint64_t>(1, 3 * S * SI / 32);

@@ -25,4 +25,12 @@ int grow_buffer(T **p, size_t *cap, size_t need, std::vector<void *> &retired, A
     return 0;
 }
 
+// The same with room for `want` >= need elements where that fits, so that calls
+// that grow a little at a time do not each retire a buffer.
+template <typename T, typename Alloc>
+int grow_stepped(T **p, size_t *cap, size_t need, size_t want, std::vector<void *> &retired, Alloc alloc) {
+    if (*cap >= need || grow_buffer(p, cap, want, retired, alloc) == 0) return 0;
+    return want > need ? grow_buffer(p, cap, need, retired, alloc) : -1;
+}
+
 }  // namespace cz

@@ -229,6 +229,36 @@ static void scratch_cases() {
     for (size_t i = 0; i < cap; ++i) o[i] = 1.0f;
     for (void *q : retired) std::free(q);
     std::free(o);
+    // prompts that grow: the O rows past 8192 slots come in steps, so what they
+    // leave behind stays below what they hold, and the plan counts the step
+    retired.clear();
+    o = nullptr;
+    cap = 0;
+    left = ~(size_t)0;
+    const colizig_dims d{256, 64, 8, 128, 0, 1};
+    size_t held = 0;
+    for (uint64_t S = 1025; S <= 8192; S += 100) {
+        const uint64_t sk = S * d.topk, rows = cz::grouped_o_slots(sk);
+        CHECK(rows >= sk && rows <= cz::kPlanWideSlots);
+        const size_t before = left;
+        CHECK(cz::grow_stepped(&o, &cap, sk, rows, retired, alloc) == 0 && cap >= sk);
+        held += before - left;
+        CHECK(cz::work_bytes(d, S, true) >= 4 * (rows + 3 * S) * d.hidden);
+    }
+    CHECK(held <= 2 * cap * sizeof(float) && retired.size() <= 2);
+    CHECK(cz::grouped_o_slots(8192) == 8192 && cz::grouped_o_slots(65537) == 65537);
+    for (void *q : retired) std::free(q);
+    retired.clear();
+    std::free(o);
+    // no room for the step: the exact size, and no new request while that is enough
+    o = nullptr;
+    cap = 0;
+    left = 4 * 9000;
+    CHECK(cz::grow_stepped(&o, &cap, 8800, cz::grouped_o_slots(8800), retired, alloc) == 0 && cap == 8800);
+    calls = 0;
+    CHECK(cz::grow_stepped(&o, &cap, 8800, cz::grouped_o_slots(8800), retired, alloc) == 0 && calls == 0);
+    CHECK(cz::grow_stepped(&o, &cap, 8900, cz::grouped_o_slots(8900), retired, alloc) == -1 && cap == 8800 && o);
+    std::free(o);
 }
 
 static void plan_cases() {
