@@ -99,6 +99,7 @@ SIGNATURES = {
     "colizig_hip_fused_predict_stats": (ctypes.c_int, [ctypes.c_void_p]),
     "colizig_hip_fused_placement": (ctypes.c_int, []),
     "colizig_hip_set_fused_fault": (ctypes.c_int, [ctypes.c_int]),
+    "colizig_hip_set_scratch_limit": (ctypes.c_uint64, [ctypes.c_uint64]),
     "colizig_hip_fused_decode_active": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int]),
     "colizig_hip_chain_fused_times": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_uint32, vp, ctypes.c_float,
                                                      ctypes.c_int, vp]),

@@ -272,6 +272,7 @@ struct Ctx {
     std::unordered_map<uint32_t, LayerHost> layers;
     Work work;
     std::vector<void *> retired;
+    uint64_t scratch_limit = 0;  // colizig_hip_set_scratch_limit
     std::unordered_map<int64_t, hipGraphExec_t> graphs;
     std::unordered_map<int64_t, hipGraph_t> graph_defs;
     // (layer, generation) of every layer a graph captured
@@ -327,7 +328,9 @@ int ensure_host(size_t need) {
 
 void *dev_alloc(size_t bytes) {
     void *q = nullptr;
-    if (hipMalloc(&q, bytes) == hipSuccess) return q;
+    const bool got = hipMalloc(&q, bytes) == hipSuccess;  // asked for even past the test hook's limit, as a full device is
+    if (got && (!g.scratch_limit || bytes <= g.scratch_limit)) return q;
+    if (got) (void)hipFree(q);
     (void)hipGetLastError();  // the caller may go on without: it is no launch's error
     return nullptr;
 }
@@ -424,11 +427,16 @@ bool use_grouped(const colizig_dims &d, int S) {
            w.cap_o >= sk * d.hidden && w.cap_os >= s * d.hidden;
 }
 
-// The grouped regime's scratch, where a call of S tokens takes it.
-int ensure_grouped(const colizig_dims &d, int S) {
-    if (!grouped_ok(d, S)) return 0;
-    const int rc = ensure_work_grouped(d, S);
-    return grouped_f32x(d, S) ? 0 : rc;
+// The grouped regime's scratch, where a call of S tokens on st takes it.  A call
+// past CZ_DISPATCH_MAX slots can do without, so nothing is allocated for it
+// while st captures (that would end the capture).
+int ensure_grouped(const colizig_dims &d, int S, hipStream_t st) {
+    if (!grouped_ok(d, S) || (grouped_f32x(d, S) && use_grouped(d, S))) return 0;
+    if (!grouped_f32x(d, S)) return ensure_work_grouped(d, S);
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    CZ_CHECK(hipStreamIsCapturing(st, &cs), -4);
+    if (cs == hipStreamCaptureStatusNone) (void)ensure_work_grouped(d, S);
+    return 0;
 }
 
 void free_layer(LayerHost &L) {
@@ -2008,7 +2016,7 @@ extern "C" int colizig_hip_moe_forward_dev(uint32_t layer, const float *x_dev, i
     int rc = check_layer_ready(L, layer);
     if (rc) return rc;
     if ((rc = ensure_work(L->d, S))) return rc;
-    if ((rc = ensure_grouped(L->d, S))) return rc;
+    if ((rc = ensure_grouped(L->d, S, pick_stream(stream)))) return rc;
     if (L->streamed()) {
         if ((rc = ensure_work_grouped(L->d, S)) || (rc = ensure_h_idx(S))) return rc ? rc : -2;
         rc = run_streamed_layer(*L, layer, x_dev, S, out_dev, 0, 0.0f, nullptr, nullptr, 0, pick_stream(stream),
@@ -2127,7 +2135,7 @@ extern "C" int colizig_hip_moe_forward(uint32_t layer, const float *x, int S, fl
     int rc = check_layer_ready(L, layer);
     if (rc) return rc;
     if ((rc = ensure_work(L->d, S))) return rc;
-    if ((rc = ensure_grouped(L->d, S))) return rc;
+    if ((rc = ensure_grouped(L->d, S, g.stream))) return rc;
     const size_t xb = (size_t)S * L->d.hidden * sizeof(float);
     const size_t kb = (size_t)S * L->d.topk * sizeof(float);
     if (ensure_host(xb + 2 * kb)) return -2;
@@ -2164,7 +2172,7 @@ static int chain_enqueue(uint32_t layer0, uint32_t nlayers, float *x_dev, int S,
             return -1;
         }
         if ((rc = ensure_work(L->d, S))) return rc;
-        if ((rc = ensure_grouped(L->d, S))) return rc;
+        if ((rc = ensure_grouped(L->d, S, st))) return rc;
     }
     const int fz = chain_fused_prepare(layer0, nlayers, S);
     if (fz < 0) return fz;
@@ -2205,7 +2213,7 @@ extern "C" int64_t colizig_hip_chain_graph_create(uint32_t layer0, uint32_t nlay
         int rc = check_layer_ready(L, layer0 + l);
         if (rc) return rc;
         if ((rc = ensure_work(L->d, S))) return rc;
-        if ((rc = ensure_grouped(L->d, S))) return rc;
+        if ((rc = ensure_grouped(L->d, S, g.stream))) return rc;
     }
     if (const int fz = chain_fused_prepare(layer0, nlayers, S); fz < 0) return fz;
     CZ_CHECK(hipStreamSynchronize(g.stream), -4);
@@ -2438,7 +2446,7 @@ extern "C" int colizig_hip_chain_kernel_times(uint32_t layer0, uint32_t nlayers,
         if (rc) return rc;
         if (L->streamed()) return -1;
         if ((rc = ensure_work(L->d, S))) return rc;
-        if ((rc = ensure_grouped(L->d, S))) return rc;
+        if ((rc = ensure_grouped(L->d, S, g.stream))) return rc;
     }
     std::vector<StepArgs> args;
     for (uint32_t l = 0; l < nlayers; ++l) {
@@ -3930,6 +3938,15 @@ extern "C" int colizig_hip_set_fused_fault(int pos) {
     std::lock_guard<std::recursive_mutex> lk(g_mu);
     const int prev = g.fused.fault_pos;
     g.fused.fault_pos = pos < 0 ? -1 : pos;
+    return prev;
+}
+
+// Test hook: scratch buffers of more than this many bytes are refused as on a
+// full device (0: no limit).  Returns the previous limit.
+extern "C" uint64_t colizig_hip_set_scratch_limit(uint64_t bytes) {
+    std::lock_guard<std::recursive_mutex> lk(g_mu);
+    const uint64_t prev = g.scratch_limit;
+    g.scratch_limit = bytes;
     return prev;
 }
 

@@ -273,6 +273,11 @@ int colizig_hip_fused_placement(void);
  * position.  No counterpart in the reference. */
 int colizig_hip_set_fused_fault(int pos);
 
+/* Test hook: scratch buffers of more than `bytes` are refused as on a full
+ * device (0, the default: no limit); returns the previous limit.  No
+ * counterpart in the reference. */
+uint64_t colizig_hip_set_scratch_limit(uint64_t bytes);
+
 /* The grouped regime's GEMMs (prefill, batch decode) on FP8 MFMA
  * (v_mfma_scale_f32_32x32x64_f8f6f4: E4M3 weights as they are, the A rows as
  * three E4M3 terms with E8M0 exponents per 32 columns; the default) when
