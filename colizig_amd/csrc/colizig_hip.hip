@@ -403,7 +403,7 @@ int ensure_work_grouped(const colizig_dims &d, int S) {
 // calls have always had (k_gg_f32x; the forms that split the rows beforehand
 // hold 12 or 22 bits), up to kPlanWideSlots: their O rows are 4 H bytes a slot
 // (0.5 GB at 65,536 slots of 2048).  2000 tokens of a Qwen3-30B-A3B layer
-// (16,000 slots): 10,800 us with the per-token kernels, 555 us.
+// (16,000 slots): 10,800 us with the per-token kernels, 630 us.
 bool grouped_f32x(const colizig_dims &d, int S) {
     const size_t sk = (size_t)S * d.topk;
     return sk > CZ_DISPATCH_MAX && sk <= cz::kPlanWideSlots;
@@ -1540,17 +1540,17 @@ void launch_gemm_f32x_t(GemvMulti G, const float *x, int S, int I, hipStream_t s
     k_gemm_f32x<MR, WN, KS><<<(items + 7) / 8 * 8, 64 * WN * KS, 0, st>>>(G, x, (uint32_t)S, (uint32_t)I);
 }
 
-// Many-token products on the f16 matrix cores (k_gemm_f32x).  The rule looks at
+// Many-token products on the bf16 matrix cores (k_gemm_f32x).  The rule looks at
 // S and I alone, so that a matrix has the same bits in any launch.
 //
-// The GEMV's time grows with S, the products' hardly up to 96 tokens (16-row
-// tiles, K over four waves): 2048 columns 11 us against 14 (512 rows) and 21
-// (4096) at 16 tokens, 11 against 11 and 17 at 12; 4096 columns 19 against 23
-// (2048 rows) and 37 (4096) at 8, 512 columns 5.5 against 5.7 at 16.  From 129
-// tokens K goes over two wave groups and twice the columns (q, k, v and o: 128
-// tokens 41 against 45 us, 160 tokens 52 against 46, 385 tokens 95 against 71;
-// 32-row tiles 81 there), from 513 four waves stand side by side on 32-row
-// tiles (1000 tokens 127 us, K over two wave groups 139).
+// The GEMV's time grows with S, the products' hardly up to 128 tokens (16-row
+// tiles, K over four waves): 2048 columns 11 us against 14 (512 rows) and 28 (q,
+// k and v) at 16 tokens, 4096 columns 20 against 21 (512 rows) and 23 (2048) at 8,
+// 512 columns 5.7 against 6.1 at 16.  Beyond, K goes over two wave groups and
+// twice the columns (us for q, k, v and for o: 192 tokens 27 and 25 against 22
+// and 29, 320 45 and 41 against 40 and 39, 512 65 and 51 against 52 and 40); from
+// 513 four waves stand side by side on 32-row tiles (there 58 and 61 against 47
+// and 66, 1000 tokens 97 and 77 against 83 and 68).
 constexpr int kGemmF32xShortTokens = 128, kGemmF32xSplitTokens = 512;
 bool launch_gemm_f32x(const GemvMulti &G, const float *x, int S, int I, hipStream_t st) {
     if (I % CZ_BLOCK || (S < 16 && (int64_t)S * I < 28672)) return false;

@@ -1,30 +1,84 @@
-// cz_gemm.h - E4M3 weights times f32 rows on the f16 matrix cores at f32's
-// accuracy: many-token projections (matmulFp8, fp8.zig:215-257) and the
+// cz_gemm.h - E4M3 weights times f32 rows on the bf16 matrix cores with every
+// bit of the rows: many-token projections (matmulFp8, fp8.zig:215-257) and the
 // grouped expert products of prompts past the FP8 form's slots.
 //
-// A K block of a row (128 columns, one weight scale block) is multiplied by a
-// power of two that puts its largest element in [2^14, 2^15), then split as
-// f16 hi + lo: hi keeps 11 bits, lo the next 11, so at most the last bit of an
-// f32 is rounded, and elements down to 2^-16 of the largest keep all of it (no
-// f16 subnormals).  E4M3 is exact in f16, every product is exact in f32, and
-// each K block's sum is taken alone and then added as tot = fma(blk 2^e, s,
-// tot) with the block scale s (the product with 2^e is exact).
+// An f32 is the sum of three bf16 numbers, each the upper half of what is left
+// (8 significant bits at f32's exponent range), and E4M3 is exact in bf16.  So
+// every product is exact, a K block (128 columns, one weight scale block) is
+// summed in f32 alone and added as tot = fma(blk, s, tot): the f32 kernels'
+// products and sums, in another order.  The
+// rows are scaled by 2^16 and the weights by 2^-16 on the way, because a bf16
+// subnormal ends at 2^-133 where an f32 ends at 2^-149.  Row blocks with an
+// element of 2^100 or more are scaled by 1/2 instead (no block sum overflows)
+// and flagged: of those, bits below 2^-132 are lost.
 //
-// The split is done as the rows are staged in LDS, so no pass before the
-// product and no scratch is needed, and the f32 row is as many bytes as hi and
-// lo together.
+// The split is done as the rows are staged in LDS, or, where a single wave reads
+// a staged row, as it reads it: no pass before the product and no scratch.
 //
-// Bound: one K block of a 32 x 256 tile is 1,024 cycles of MFMA a SIMD beside
-// about as many of vector work (the split, E4M3 to f16, the fold into tot) and
-// of LDS traffic; two workgroups on a CU overlap them to about 3,200 cycles,
-// one alone takes 4,000.  Measured and not kept: loads two K blocks ahead (the
-// same time: the loads are not what is waited for), 64-row tiles with eight
-// waves (1500 tokens' q, k, v 103-172 against 84 us).
+// Bound: one K block of a 32 x 256 tile is 1,536 cycles of MFMA a SIMD.  In the
+// gate/up products of 2000 tokens (two workgroups a CU) the counters give 45% of
+// the time in MFMA, each of a SIMD's two waves 23% in vector work (E4M3 to bf16,
+// the split, the sums) and 18% waiting for memory or a barrier, and the LDS 30%
+// busy: vector work and MFMA hardly overlap.  Two f16 terms (hi + lo, 23 bits, and
+// fewer beside elements 2^16 times larger) took 555 us where the layer takes 630;
+// the error against 64 bits is 2.2e-7 for 2.4e-7, and of the projections at 385
+// tokens 0.9e-7 for 1.3e-7 (the GEMV's: 1.6e-7).  Measured and not kept: loads two
+// K blocks ahead, and the weights widened one step ahead or without scheduling
+// fences (the same time or up to 4% more).
 #pragma once
 
 #include "cz_grouped.h"
 
-#define CZ_GF_ALD 272  // LDS bytes per staged K block of a row (256 + 16: rows in distinct bank groups)
+typedef __bf16 cz_bf8 __attribute__((ext_vector_type(8)));
+
+#define CZ_GF_UP 0x1p16f     // scale of the rows, undone by the weights'
+#define CZ_GF_BIG 0x1p100f   // from here on a row block is scaled by
+#define CZ_GF_DOWN 0x1p-1f   // this, and its sums by
+#define CZ_GF_F 0x1p17f      // this
+
+// 8 E4M3 bytes -> 8 bf16, times 2^-16, exact (0x7F: NaN).
+__device__ __forceinline__ cz_bf8 cz_fp8x8_to_bf16(uint32_t w0, uint32_t w1) {
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    constexpr float sc = 1.0f / CZ_GF_UP;
+    const bf2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w0, sc, false);
+    const bf2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w0, sc, true);
+    const bf2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w1, sc, false);
+    const bf2 p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w1, sc, true);
+    cz_bf8 r;
+    r[0] = p0[0]; r[1] = p0[1]; r[2] = p1[0]; r[3] = p1[1];
+    r[4] = p2[0]; r[5] = p2[1]; r[6] = p3[0]; r[7] = p3[1];
+    return r;
+}
+
+// v = hi + mid + lo, each as words of two bf16.  inf (wave-uniform): there may be
+// infinities, which have no lower parts (inf - inf); a NaN stays one in some part.
+template <int N>
+__device__ __forceinline__ void cz_bf16_split(const float (&v)[N], bool inf, uint32_t (&hi)[N / 2],
+                                              uint32_t (&mid)[N / 2], uint32_t (&lo)[N / 2]) {
+    float r[N];
+    auto take = [&](uint32_t(&out)[N / 2]) {  // the upper halves
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i)
+            out[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, r[2 * i + 1]),
+                                           __builtin_bit_cast(uint32_t, r[2 * i]), 0x07060302u);
+    };
+    auto rest = [&] {  // what they leave, exactly
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            r[i] = r[i] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r[i]) & 0xffff0000u);
+    };
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i] = v[i];
+    take(hi);
+    rest();
+    if (inf)
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (__builtin_isinf(v[i])) r[i] = 0.0f;
+    take(mid);
+    rest();
+    take(lo);
+}
 
 // One wave's part of a tile: MR rows x 64 weight rows, as 32 x 32 x 16 products
 // (MR = 32: two subtiles) or 16 x 16 x 32 ones (MR = 16: four).  Lane l holds
@@ -38,26 +92,31 @@ struct GFWave {
     __device__ static __forceinline__ uint32_t row(uint32_t lane, int i) {
         return MR == 32 ? (i / 4) * 8u + (lane >> 5) * 4u + (i % 4) : (lane >> 4) * 4u + i;
     }
-    __device__ static __forceinline__ V mfma(cz_half8 a, cz_half8 b, V c) {
+    __device__ static __forceinline__ V mfma(cz_bf8 a, cz_bf8 b, V c) {
         if constexpr (MR == 32)
-            return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+            return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
         else
-            return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }
 };
 
 // One workgroup's tile: its WN x KS waves take the same MR rows and 64 weight
 // rows each; KS wave groups take every KS-th K block and their sums are added
-// at the end.
+// at the end.  RAW (one wave reads a staged row): the rows are staged as f32
+// and split where they are read, which keeps two workgroups on a CU; else each
+// is split once for the waves that share it.
 template <int MR, int WN, int KS>
 struct GFLds {
-    static constexpr int RB = MR * KS;  // K blocks of rows staged per pass
-    uint8_t hi[RB * CZ_GF_ALD];
-    uint8_t lo[RB * CZ_GF_ALD];
+    static constexpr bool RAW = WN == 1;
+    static constexpr int RB = MR * KS;                  // K blocks of rows staged per pass
+    static constexpr int ALD = RAW ? 512 + 16 : 256 + 16;  // LDS bytes of each (+ 16: rows in distinct bank groups)
+    static constexpr int PLANES = RAW ? 1 : 3;
+    uint8_t a[PLANES][RB * ALD];
     uint8_t w[WN * KS][64 * CZ_GG_WLD];
-    float f[RB];       // 2^e that undoes each row block's scaling
-    uint64_t src[MR];  // element offset of each tile row's A row
-    uint32_t dst[MR];  // C row, ~0u: padding
+    float f[RB];               // undoes the scaling of a flagged pass's row blocks
+    uint32_t big[WN * KS];     // staging wave saw an element of CZ_GF_BIG or more
+    uint64_t src[MR];          // element offset of each tile row's A row
+    uint32_t dst[MR];          // C row, ~0u: padding
 };
 
 // tot = the wave's products: weight rows 0-31 are wb[0]'s, 32-63 wb[1]'s (each
@@ -68,6 +127,7 @@ __device__ __forceinline__ void cz_gf_tile(GFLds<MR, WN, KS> &sh, const float *_
                                            const float *const (&sr)[2],
                                            typename GFWave<MR>::V (&tot)[GFWave<MR>::NSUB]) {
     typedef GFWave<MR> W;
+    typedef GFLds<MR, WN, KS> L;
     typedef typename W::V V;
     constexpr int NT = 64 * WN * KS, RB = MR * KS;
     constexpr int NA = RB * 16 / NT;  // row blocks per thread (16 lanes each, two float4 a lane)
@@ -111,73 +171,82 @@ __device__ __forceinline__ void cz_gf_tile(GFLds<MR, WN, KS> &sh, const float *_
     auto store = [&] {
 #pragma unroll
         for (int p = 0; p < NW; ++p) *(u32x4 *)(wst + p * 8 * CZ_GG_WLD) = wv[p];
-        float mx[NA];
+        float all = 0.0f, up[NA];
 #pragma unroll
         for (int p = 0; p < NA; ++p) {
-            const float *v = (const float *)av[p];
-            mx[p] = 0.0f;
+            up[p] = CZ_GF_UP;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) mx[p] = fmaxf(mx[p], __builtin_fabsf(v[i]));
+            for (int i = 0; i < 8; ++i) all = fmaxf(all, __builtin_fabsf(((const float *)av[p])[i]));
         }
+        const bool big = __builtin_amdgcn_ballot_w64(all >= CZ_GF_BIG) != 0;  // infinities too
+        if (big) {
 #pragma unroll
-        for (int p = 0; p < NA; ++p) mx[p] = fmaxf(mx[p], cz_dpp<0xB1>(mx[p]));
+            for (int p = 0; p < NA; ++p) {
+                float mx = 0.0f;
 #pragma unroll
-        for (int p = 0; p < NA; ++p) mx[p] = fmaxf(mx[p], cz_dpp<0x4E>(mx[p]));
-#pragma unroll
-        for (int p = 0; p < NA; ++p) mx[p] = fmaxf(mx[p], cz_dpp<0x141>(mx[p]));
-#pragma unroll
-        for (int p = 0; p < NA; ++p) mx[p] = fmaxf(mx[p], cz_dpp<0x140>(mx[p]));
-        bool inf = false;
-        cz_half4 h[NA][2], l[NA][2];
+                for (int i = 0; i < 8; ++i) mx = fmaxf(mx, __builtin_fabsf(((const float *)av[p])[i]));
+                mx = fmaxf(mx, cz_dpp<0xB1>(mx));
+                mx = fmaxf(mx, cz_dpp<0x4E>(mx));
+                mx = fmaxf(mx, cz_dpp<0x141>(mx));
+                mx = fmaxf(mx, cz_dpp<0x140>(mx));
+                if (mx >= CZ_GF_BIG) up[p] = CZ_GF_DOWN;
+            }
+        }
+        if (lane == 0) sh.big[wave] = big;
 #pragma unroll
         for (int p = 0; p < NA; ++p) {
-            // 2^(141 - E) and its inverse, E the biased exponent (at least 15, so
-            // that both are normal); an infinity (E = 255) scales the rest down too
-            const uint32_t E = max(__builtin_bit_cast(uint32_t, mx[p]) >> 23, 15u);
-            const float up = __builtin_bit_cast(float, (268u - E) << 23);
-            if (q == 0) sh.f[(tid >> 4) + p * (NT / 16)] = __builtin_bit_cast(float, (E - 14u) << 23);
-            inf |= E == 255u;
-            const float *v = (const float *)av[p];
+            const uint32_t rb = (tid >> 4) + p * (NT / 16);
+            if (q == 0) sh.f[rb] = up[p] == CZ_GF_UP ? 1.0f : CZ_GF_F;
+            float v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const _Float16 hi = (_Float16)(v[i] * up);
-                h[p][i / 4][i % 4] = hi;
-                l[p][i / 4][i % 4] = (_Float16)__builtin_fmaf(v[i], up, -(float)hi);  // exact, then rounded
+            for (int i = 0; i < 8; ++i) v[i] = ((const float *)av[p])[i] * up[p];
+            if constexpr (L::RAW) {
+                uint8_t *o = sh.a[0] + rb * L::ALD + 16 * q;
+                *(float4 *)o = make_float4(v[0], v[1], v[2], v[3]);
+                *(float4 *)(o + 256) = make_float4(v[4], v[5], v[6], v[7]);
+            } else {
+                uint32_t t[3][4];
+                cz_bf16_split(v, big, t[0], t[1], t[2]);
+#pragma unroll
+                for (int k = 0; k < L::PLANES; ++k) {
+                    uint8_t *o = sh.a[k] + rb * L::ALD + 8 * q;
+                    *(uint2 *)o = make_uint2(t[k][0], t[k][1]);
+                    *(uint2 *)(o + 128) = make_uint2(t[k][2], t[k][3]);
+                }
             }
         }
-        if (inf) {  // inf - inf: an infinity has no lower part
-#pragma unroll
-            for (int p = 0; p < NA; ++p)
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (__builtin_isinf(((const float *)av[p])[i])) l[p][i / 4][i % 4] = (_Float16)0.0f;
-        }
-#pragma unroll
-        for (int p = 0; p < NA; ++p)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const uint32_t o = ((tid >> 4) + p * (NT / 16)) * CZ_GF_ALD + 8 * q + 128 * i;
-                *(cz_half4 *)(sh.hi + o) = h[p][i];
-                *(cz_half4 *)(sh.lo + o) = l[p][i];
-            }
     };
     const uint32_t rl = lane & (MR - 1), kg = lane / MR;
-    const uint32_t ao = (kh * MR + rl) * CZ_GF_ALD + kg * (256 / W::G);  // + 16 s
-    const uint8_t *lr = lw + rl * CZ_GG_WLD + kg * (128 / W::G);         // + 8 s: the same K order
+    const uint32_t ao = (kh * MR + rl) * L::ALD + kg * ((L::RAW ? 512 : 256) / W::G);  // + 8 s elements
+    const uint8_t *lr = lw + rl * CZ_GG_WLD + kg * (128 / W::G);                       // + 8 s: the same K order
+    static_assert(WN * KS == 4, "the staging waves' flags are one 16-byte word");
     auto multiply = [&](uint32_t it) {
         const uint32_t kb = it * KS + kh;
         if (KS > 1 && kb >= nkb) return;  // wave-uniform
         const float sc[2] = {cz_const_f32(sr[0] + kb), cz_const_f32(sr[1] + kb)};
+        const uint4 bg = *(const uint4 *)sh.big;
+        const bool big = __builtin_amdgcn_readfirstlane((int)(bg.x | bg.y | bg.z | bg.w)) != 0;
         V blk[W::NSUB] = {}, low[W::NSUB] = {};
         u32x4 wq[2][W::NSUB];
-        cz_half8 xh[2], xl[2];
+        cz_bf8 xt[2][3];
         auto fetch_w = [&](int s2) {
 #pragma unroll
             for (int m = 0; m < W::NSUB; ++m) wq[s2 & 1][m] = *(const u32x4 *)(lr + m * MR * CZ_GG_WLD + 16 * s2);
         };
         auto fetch_a = [&](int s) {
-            xh[s & 1] = *(const cz_half8 *)(sh.hi + ao + 16 * s);
-            xl[s & 1] = *(const cz_half8 *)(sh.lo + ao + 16 * s);
+            if constexpr (L::RAW) {
+                float v[8];
+                *(float4 *)&v[0] = *(const float4 *)(sh.a[0] + ao + 32 * s);
+                *(float4 *)&v[4] = *(const float4 *)(sh.a[0] + ao + 32 * s + 16);
+                uint32_t t[3][4];
+                cz_bf16_split(v, big, t[0], t[1], t[2]);
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    xt[s & 1][k] = __builtin_bit_cast(cz_bf8, u32x4{t[k][0], t[k][1], t[k][2], t[k][3]});
+            } else {
+#pragma unroll
+                for (int k = 0; k < L::PLANES; ++k) xt[s & 1][k] = *(const cz_bf8 *)(sh.a[k] + ao + 16 * s);
+            }
         };
         fetch_w(0);
         fetch_a(0);
@@ -186,35 +255,33 @@ __device__ __forceinline__ void cz_gf_tile(GFLds<MR, WN, KS> &sh, const float *_
         for (int s = 0; s < W::NS; ++s) {  // step s + 1's operands are read while step s multiplies
             if (s + 1 < W::NS) fetch_a(s + 1);
             if (s >= 2 && s % 2 == 0 && s / 2 + 1 < W::NS / 2) fetch_w(s / 2 + 1);
-            cz_half8 b[W::NSUB];
+            cz_bf8 b[W::NSUB];
 #pragma unroll
             for (int m = 0; m < W::NSUB; ++m) {
                 const u32x4 w = wq[(s >> 1) & 1][m];
-                b[m] = (s & 1) ? cz_fp8x8_to_f16(w[2], w[3]) : cz_fp8x8_to_f16(w[0], w[1]);
+                b[m] = (s & 1) ? cz_fp8x8_to_bf16(w[2], w[3]) : cz_fp8x8_to_bf16(w[0], w[1]);
             }
+            // the lower parts' sum is rounded into the rest once
 #pragma unroll
-            for (int m = 0; m < W::NSUB; ++m)
-                if constexpr (KS == 1)
-                    low[m] = W::mfma(xl[s & 1], b[m], low[m]);
-                else
-                    blk[m] = W::mfma(xl[s & 1], b[m], blk[m]);
+            for (int m = 0; m < W::NSUB; ++m) low[m] = W::mfma(xt[s & 1][2], b[m], low[m]);
 #pragma unroll
-            for (int m = 0; m < W::NSUB; ++m) blk[m] = W::mfma(xh[s & 1], b[m], blk[m]);
+            for (int m = 0; m < W::NSUB; ++m) low[m] = W::mfma(xt[s & 1][1], b[m], low[m]);
+#pragma unroll
+            for (int m = 0; m < W::NSUB; ++m) blk[m] = W::mfma(xt[s & 1][0], b[m], blk[m]);
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int m = 0; m < W::NSUB; ++m)
-            if constexpr (KS == 1) blk[m] += low[m];  // the low parts' sum is rounded into the rest once
+        for (int m = 0; m < W::NSUB; ++m) blk[m] += low[m];
+        if (big) {
 #pragma unroll
-        for (int j = 0; j < W::NV / 4; ++j) {
-            const float4 f4 = *(const float4 *)(sh.f + kh * MR + W::row(lane, 4 * j));
-            const float f[4] = {f4.x, f4.y, f4.z, f4.w};
+            for (int i = 0; i < W::NV; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int m = 0; m < W::NSUB; ++m)
-                    tot[m][4 * j + i] = __builtin_fmaf(blk[m][4 * j + i] * f[i], sc[m * MR / 32], tot[m][4 * j + i]);
+                for (int m = 0; m < W::NSUB; ++m) blk[m][i] *= sh.f[kh * MR + W::row(lane, i)];
         }
+#pragma unroll
+        for (int i = 0; i < W::NV; ++i)
+#pragma unroll
+            for (int m = 0; m < W::NSUB; ++m) tot[m][i] = __builtin_fmaf(blk[m][i], sc[m * MR / 32], tot[m][i]);
     };
 #pragma unroll
     for (int m = 0; m < W::NSUB; ++m) tot[m] = V{};
@@ -251,8 +318,7 @@ __device__ __forceinline__ void cz_gf_tile(GFLds<MR, WN, KS> &sh, const float *_
 // y_m[S][O_m] = x[S][I] . dequant(W_m)^T, I % 128 == 0: MR rows x 64 WN
 // columns per workgroup.  Item t of the launch is column tile t / mtiles, row
 // tile t % mtiles; each XCD (block % 8) walks a contiguous range, so a column
-// tile's weights are read into one XCD's L2 once.  Error against 64 bits at the
-// Qwen3-30B-A3B projections 1.2-1.3e-7 (the GEMV's: 1.6e-7).
+// tile's weights are read into one XCD's L2 once.
 template <int MR, int WN, int KS>
 __global__ __launch_bounds__(64 * WN * KS, 2) void k_gemm_f32x(GemvMulti G, const float *__restrict__ x, uint32_t S,
                                                                   uint32_t I) {
@@ -305,8 +371,8 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void k_gemm_f32x(GemvMulti G, cons
 // subtiles are the gate and up rows of the same 32 outputs, h = silu(g) u as
 // f32; DOWN: 64 adjacent rows.  The shared expert's items (PS) run first in the
 // same launch; items and their XCD ranges as in k_gg.  2000 tokens of a
-// Qwen3-30B-A3B layer, Zipf(1.1): gate/up 313 us, down 177 us; the layer's
-// error against 64 bits 2.4e-7 (the per-token kernels': 2.6e-7).
+// Qwen3-30B-A3B layer, Zipf(1.1): gate/up 425 us, down 230 us (medians of the
+// kernel trace).
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void k_gg_f32x(GroupArgs G, GGProblem PR, GGProblem PS, const float *__restrict__ aR,
                                                     const float *__restrict__ aS) {

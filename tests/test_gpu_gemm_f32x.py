@@ -2,10 +2,10 @@
 64-bit sums over tile edges, odd rows and columns, wide ranges of magnitude,
 infinities and NaN; and layers past 8192 slots against the oracle.
 
-The bound on the relative L2 error: the f16 hi + lo split keeps 2^-24 of each
-element, a K block's 128 exact products are summed in f32 (at most 24 rounded
-additions, random signs: about sqrt(24) 2^-25), then one FMA per K block:
-about 2e-7 in all; 6e-7 is asserted."""
+The bound on the relative L2 error: the split into three bf16 terms is exact, a
+K block's 128 exact products are summed in f32 (at most 24 rounded additions,
+random signs: about sqrt(24) 2^-25), then one FMA per K block: about 2e-7 in
+all; 6e-7 is asserted."""
 from __future__ import annotations
 
 import numpy as np
@@ -86,7 +86,7 @@ def test_many_tokens_f32_accuracy(gpu, S, I, Os):
         moe.set_vram_budget(0)
 
 
-@pytest.mark.parametrize("S", [16, 40])
+@pytest.mark.parametrize("S", [16, 40, 129, 513])
 def test_extreme_values(gpu, S):
     """Infinities, NaN, zero rows, the largest and smallest floats, a NaN
     weight and a zero scale: what f32 sums of the same products give."""
@@ -115,6 +115,34 @@ def test_extreme_values(gpu, S):
         assert np.array_equal(y[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
         # all terms of one sign: no cancellation
         assert (np.abs(y[fin] - ref[fin]) <= 2e-6 * np.abs(ref[fin]) + 1e-44).all()
+    finally:
+        moe.set_vram_budget(0)
+
+
+@pytest.mark.parametrize("S,I", [(16, 2048), (129, 512), (513, 384), (24, 896)])
+def test_small_elements_beside_large_ones(gpu, S, I):
+    """Each row's 128-column blocks hold one element 1e6 to 1e30 times the
+    rest, whose weights are zero: the result is the rest's, with all of their
+    bits, as f32 sums give it.  Rows of the smallest floats keep theirs too."""
+    rng = np.random.default_rng(S + I)
+    O = 200
+    moe.set_vram_budget(1 << 30)
+    try:
+        w, s = synth.block_quantize(rng.normal(0, 0.02, size=(O, I)).astype(np.float32))
+        w[:, 5::128] = 0
+        x = rng.normal(size=(S, I)).astype(np.float32)
+        ratio = 10.0 ** np.array([6, 8, 10, 15, 20, 30])[np.arange(S) % 6]
+        x[:, 5::128] = ratio[:, None] * rng.choice([-1.0, 1.0], size=(S, len(range(5, I, 128))))
+        tiny = np.arange(S) % 8 == 7
+        x[tiny] = 1e-37 * rng.normal(size=(int(tiny.sum()), I))  # down to subnormals; none beside them
+        key = moe.Fp8Matrix.expert_key(71, S % 500, 1)
+        moe.matrix_load(key, w, s)
+        y = _run(x, [(w, s, key)], I)[0]
+        ref = x.astype(np.float64) @ _dequant(w, s).T
+        err = np.linalg.norm(y - ref, axis=1) / np.linalg.norm(ref, axis=1)
+        print(f"small beside large S={S} I={I}: worst row {err.max():.2e}", flush=True)
+        assert err[~tiny].max() < RTOL
+        assert err[tiny].max() < 1e-6  # results near 5e-38, whose last place is 2^-149, besides
     finally:
         moe.set_vram_budget(0)
 
