@@ -273,10 +273,22 @@ __device__ __forceinline__ void cz_gf_tile(GFLds<MR, WN, KS> &sh, const float *_
 #pragma unroll
         for (int m = 0; m < W::NSUB; ++m) blk[m] += low[m];
         if (big) {
+            // the factor goes to the scale where that is at most 1, else to the sum:
+            // neither overflows unless the term does
 #pragma unroll
-            for (int i = 0; i < W::NV; ++i)
+            for (int i = 0; i < W::NV; ++i) {
+                const float f = sh.f[kh * MR + W::row(lane, i)];
 #pragma unroll
-                for (int m = 0; m < W::NSUB; ++m) blk[m][i] *= sh.f[kh * MR + W::row(lane, i)];
+                for (int m = 0; m < W::NSUB; ++m) {
+                    const float s = sc[m * MR / 32];
+                    if (s <= 1.0f) {
+                        tot[m][i] = __builtin_fmaf(blk[m][i], s * f, tot[m][i]);
+                        blk[m][i] = 0.0f;  // added
+                    } else {
+                        blk[m][i] *= f;
+                    }
+                }
+            }
         }
 #pragma unroll
         for (int i = 0; i < W::NV; ++i)

@@ -147,6 +147,35 @@ def test_small_elements_beside_large_ones(gpu, S, I):
         moe.set_vram_budget(0)
 
 
+@pytest.mark.parametrize("S", [16, 129, 513])
+@pytest.mark.parametrize("I", [256, 384])
+def test_largest_floats(gpu, S, I):
+    """Rows whose products with the weights' bytes pass the largest float
+    where those with the scaled weights, the result's terms, do not."""
+    rng = np.random.default_rng(S + I)
+    O = 130
+    moe.set_vram_budget(1 << 30)
+    try:
+        w, s = synth.block_quantize(np.abs(rng.normal(0, 0.02, size=(O, I))).astype(np.float32) + 0.01)
+        x = np.abs(rng.normal(size=(S, I))).astype(np.float32)
+        x[0] = 3e37
+        x[3] = 1e36 * (1 + x[3])
+        x[S - 1, ::2] = 2e36
+        x[5] = 3.4e38  # its result does pass it
+        key = moe.Fp8Matrix.expert_key(72, S + I % 3, 1)
+        moe.matrix_load(key, w, s)
+        y = _run(x, [(w, s, key)], I)[0]
+        with np.errstate(all="ignore"):
+            ref = (x.astype(np.float64) @ _dequant(w, s).T).astype(np.float32)
+        assert np.isfinite(ref[:5]).all() and np.isinf(ref[5]).any()
+        near = np.abs(ref) > 3.3e38  # on either side of the limit
+        assert np.array_equal(np.isinf(y) | near, np.isinf(ref) | near) and not np.isnan(y).any()
+        fin = np.isfinite(ref) & ~near
+        assert (np.abs(y[fin] - ref[fin]) <= 2e-6 * np.abs(ref[fin])).all()
+    finally:
+        moe.set_vram_budget(0)
+
+
 @pytest.mark.parametrize("H,E,K,I,SI,S", [(256, 16, 8, 128, 0, 1025), (512, 24, 10, 256, 0, 900),
                                           (256, 64, 16, 384, 256, 600)])
 def test_layer_past_8192_slots(gpu, H, E, K, I, SI, S):
