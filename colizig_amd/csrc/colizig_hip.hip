@@ -1543,17 +1543,30 @@ void launch_gemm_f32x_t(GemvMulti G, const float *x, int S, int I, hipStream_t s
 // Many-token products on the bf16 matrix cores (k_gemm_f32x).  The rule looks at
 // S and I alone, so that a matrix has the same bits in any launch.
 //
-// The GEMV's time grows with S, the products' hardly up to 128 tokens (16-row
-// tiles, K over four waves): 2048 columns 11 us against 14 (512 rows) and 28 (q,
-// k and v) at 16 tokens, 4096 columns 20 against 21 (512 rows) and 23 (2048) at 8,
-// 512 columns 5.7 against 6.1 at 16.  Beyond, K goes over two wave groups and
-// twice the columns (us for q, k, v and for o: 192 tokens 27 and 25 against 22
-// and 29, 320 45 and 41 against 40 and 39, 512 65 and 51 against 52 and 40); from
-// 513 four waves stand side by side on 32-row tiles (there 58 and 61 against 47
-// and 66, 1000 tokens 97 and 77 against 83 and 68).
+// Up to 128 tokens (16-row tiles, K over four waves) the products' time hardly
+// depends on S.  Beyond, K goes over two wave groups and twice the columns (us for
+// q, k, v and for o: 192 tokens 27 and 25 against 22 and 29, 320 45 and 41 against
+// 40 and 39, 512 65 and 51 against 52 and 40); from 513 four waves stand side by
+// side on 32-row tiles (there 58 and 61 against 47 and 66, 1000 tokens 97 and 77
+// against 83 and 68).
 constexpr int kGemmF32xShortTokens = 128, kGemmF32xSplitTokens = 512;
+
+// The tokens from which they take over: a walk over I of about 3 + I / 240 us
+// against the GEMV's time a token, which each width's instance sets.  us of the
+// GEMV (512 rows unless said) and of the products: 512 columns
+// 6.1 / 5.7 at 16 tokens, 2048 11.3 / 11.3 at 12 and 12.9 / 11.4 at 14, 3072 14.6 /
+// 15.5 at 14 and 16.3 / 15.5 at 16, 4096 18.8 / 19.6 at 7 and 21 / 19.6 at 8; widths
+// of the generic kernel 1536 16 / 9.4 at 15, 2560 16.5 / 13.3 at 10, 3584 17.1 /
+// 17.6 at 8 and 19 / 17.5 at 9, 8192 35 / 36 at 8 and 39 / 36 at 9; 28672 16 / 116
+// at 1 and 129 / 116 at 9 (128 rows).
+int gemm_f32x_min_tokens(int I) {
+    if (I == 4096) return 8;
+    if (I == 3072) return 16;
+    return std::min(16, std::max(9, (28672 + I - 1) / I));
+}
+
 bool launch_gemm_f32x(const GemvMulti &G, const float *x, int S, int I, hipStream_t st) {
-    if (I % CZ_BLOCK || (S < 16 && (int64_t)S * I < 28672)) return false;
+    if (I % CZ_BLOCK || S < gemm_f32x_min_tokens(I)) return false;
     if (S <= kGemmF32xShortTokens)
         launch_gemm_f32x_t<16, 1, 4>(G, x, S, I, st);
     else if (S <= kGemmF32xSplitTokens)

@@ -86,6 +86,25 @@ def test_many_tokens_f32_accuracy(gpu, S, I, Os):
         moe.set_vram_budget(0)
 
 
+@pytest.mark.parametrize("S,I", [(2, 16384), (7, 14336), (7, 4096), (8, 5120), (13, 2048), (15, 3072), (15, 1024)])
+def test_fewer_tokens_keep_the_gemv(gpu, S, I):
+    """Below the products' rule the GEMV runs: a token's row has the bits it has
+    alone (the products sum in another order)."""
+    rng = np.random.default_rng(S + I)
+    O = 70
+    moe.set_vram_budget(1 << 30)
+    try:
+        w, s = synth.block_quantize(rng.normal(0, 0.02, size=(O, I)).astype(np.float32))
+        key = moe.Fp8Matrix.expert_key(73, I % 507, 1)
+        moe.matrix_load(key, w, s)
+        x = rng.normal(size=(S, I)).astype(np.float32)
+        y = _run(x, [(w, s, key)], I)[0]
+        one = np.concatenate([_run(x[t:t + 1], [(w, s, key)], I)[0] for t in range(S)])
+        assert np.array_equal(f32_bits(y), f32_bits(one))
+    finally:
+        moe.set_vram_budget(0)
+
+
 @pytest.mark.parametrize("S", [16, 40, 129, 513])
 def test_extreme_values(gpu, S):
     """Infinities, NaN, zero rows, the largest and smallest floats, a NaN
