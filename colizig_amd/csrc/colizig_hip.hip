@@ -503,15 +503,30 @@ void launch_native_mfma_t(float *y, const float *x, const uint16_t *w, int S, in
 }
 
 // BF16 rows on several tokens through the f32 matrix cores (k_native_mfma).  A
-// wave takes a whole 16-row tile, about 20 us at 2048 columns and 35-40 at 4096
+// wave takes a whole 16-row tile, about 25 us at 2048 columns and 42 at 4096
 // however few tiles there are, so the row kernel (two rows a wave) keeps the
-// small products: 16384 x 2048 at 8 tokens 34 against 25 us, 8192 x 2048 at 8
-// 17 / 25, 4096 x 2048 at 64 67 / 27; 8192 x 4096 at 8 40 / 42, 2048 x 4096 at
-// 64 106 / 41.  The tokens, in groups of four, are spread evenly over passes
-// that fit LDS (128 KiB).
-constexpr int64_t kNativeMfmaDots = 3 << 15;
+// small products.  us of the row kernel / of this one, rows x columns:
+//   from 98,304 dots on: 24576 x 2048 of 4 tokens 30 / 23, 6144 x 2048 of 16 28 / 25,
+//     512 x 2048 of 192 168 / 25, 24576 x 1024 of 4 17 / 14, 12288 x 4096 of 8 57 / 42;
+//     43691 x 1024 of 3 is the least, 21 / 24;
+//   8 to 15 tokens, up to 2048 columns: 98,304 dots are 12288 x 1024 of 8 15 / 16,
+//     8192 x 2048 of 12 23 / 28; 131,072 are 19 / 16 and 35 / 28;
+//   2 tokens: 49152 x 2048 37 / 39, 65536 x 2048 47 / 43, 151936 x 2048 119 / 115; at
+//     1024 columns 31 / 37 and 52 / 54 (98304 and 151936 rows), at 512 22 / 22 and 30 /
+//     32.
+// Widths without an instance of the row kernel (49152 x 768 of 2: 48 / 19) gain at
+// any token count.  The tokens, in groups of four, are spread evenly over passes
+// that fit LDS (128 KiB): 151936 x 2048 takes 226 us at 16 tokens and 273 at 17.
+bool native_mfma_ok(int S, int I, int O) {
+    if (S < 2 || S > 4 * 65535 || I % 256 || I > 8192) return false;
+    const int64_t dots = (int64_t)S * O;
+    const bool row_kernel = I == 256 || I == 512 || I == 1024 || I == 2048;  // and 3072, 4096
+    if (row_kernel && S == 2) return I == 2048 && dots >= 1 << 17;
+    return dots >= (row_kernel && S >= 8 && S < 16 ? 1 << 17 : 3 << 15);
+}
+
 bool launch_native_mfma(float *y, const float *x, const uint16_t *w, int S, int I, int O, hipStream_t st) {
-    if (S < 2 || S > 4 * 65535 || I % 256 || I > 8192 || (int64_t)S * O < kNativeMfmaDots) return false;
+    if (!native_mfma_ok(S, I, O)) return false;
     const int fit = std::min(4, (128 << 10) / (16 * I)), groups = (S + 3) / 4;  // fit >= 1
     const int passes = (groups + fit - 1) / fit;
     switch ((groups + passes - 1) / passes) {  // token groups of a pass, evenly
