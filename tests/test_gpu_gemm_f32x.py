@@ -61,7 +61,9 @@ def _run(xs, mats, I):
 
 @pytest.mark.parametrize("S,I,Os", [(16, 2048, (4096, 512, 512)), (31, 128, (130, 7)), (33, 384, (300,)),
                                     (64, 896, (65, 256, 1)), (385, 512, (4097, 2048)), (97, 4096, (2048,)),
-                                    (1, 2048, (512,)), (12, 2048, (512,)), (200, 768, (2048,)), (513, 512, (300, 64))])
+                                    (1, 2048, (512,)), (12, 2048, (512,)), (200, 768, (2048,)), (513, 512, (300, 64)),
+                                    (14, 2048, (200, 70)), (15, 2048, (70,)), (8, 4096, (70,)), (9, 5120, (70,)),
+                                    (128, 512, (130,)), (129, 512, (130,)), (512, 384, (130,))])
 def test_many_tokens_f32_accuracy(gpu, S, I, Os):
     print(f"f32x S={S} I={I} O={Os}", flush=True)
     rng = np.random.default_rng(S * 7 + I)
