@@ -328,7 +328,7 @@ int ensure_host(size_t need) {
 
 void *dev_alloc(size_t bytes) {
     void *q = nullptr;
-    const bool got = hipMalloc(&q, bytes) == hipSuccess;  // asked for even past the test hook's limit, as a full device is
+    const bool got = hipMalloc(&q, bytes) == hipSuccess;  // also past the test hook's limit, as a full device is asked
     if (got && (!g.scratch_limit || bytes <= g.scratch_limit)) return q;
     if (got) (void)hipFree(q);
     (void)hipGetLastError();  // the caller may go on without: it is no launch's error
@@ -402,7 +402,8 @@ int ensure_work_grouped(const colizig_dims &d, int S) {
 // Past CZ_DISPATCH_MAX slots the grouped GEMMs keep f32's accuracy, which such
 // calls have always had (k_gg_f32x; the forms that split the rows beforehand
 // hold 12 or 22 bits), up to kPlanWideSlots: their O rows are 4 H bytes a slot
-// (0.5 GB at 65,536 slots of 2048).  2000 tokens of a Qwen3-30B-A3B layer
+// (0.5 GB at 65,536 slots of 2048).  Longer calls run the per-token kernels as
+// ever, about twenty times the time a token.  2000 tokens of a Qwen3-30B-A3B layer
 // (16,000 slots): 10,800 us with the per-token kernels, 630 us.
 bool grouped_f32x(const colizig_dims &d, int S) {
     const size_t sk = (size_t)S * d.topk;
@@ -1592,7 +1593,8 @@ bool launch_gemm_f32x(const GemvMulti &G, const float *x, int S, int I, hipStrea
 }
 
 // y[S][O] = x[S][I] . dequant(W)^T on device pointers (matmulFp8's
-// contract, fp8.zig:215-257): the row-parallel GEMV for I = 64 x {4, 8, 16,
+// contract, fp8.zig:215-257): the many-token products from
+// gemm_f32x_min_tokens on, below the row-parallel GEMV for I = 64 x {4, 8, 16,
 // 32, 48, 64} (rows 16-byte aligned), else the generic kernel.
 void launch_matmul_fp8(float *y, const float *x, const uint8_t *w, const float *s, int S, int I, int O,
                        hipStream_t st) {
@@ -1755,8 +1757,8 @@ extern "C" int colizig_hip_matmul_fp8_dev(float *y_dev, const float *x_dev, int 
 
 // Several keyed FP8 matrices of one row width on the same input rows in one
 // launch: y_devs[m][S][Os[m]] = x . dequant(W_keys[m])^T, each bit-identical
-// to colizig_hip_matmul_fp8_dev of that key alone (the same per-row kernel
-// body).  For a caller that has the q, k and v projections of a layer
+// to colizig_hip_matmul_fp8_dev of that key alone (the same rule on S and I, and
+// the same kernel body).  For a caller that has the q, k and v projections of a layer
 // together (attn.zig:206-208 makes them three matmulFp8Keyed calls): one
 // launch instead of three.  n in 1..4; every key resident as FP8 [Os[m]][I].
 extern "C" int colizig_hip_matmul_fp8_dev_multi(int n, float *const *y_devs, const uint64_t *keys, const int *Os,

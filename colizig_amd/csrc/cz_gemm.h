@@ -18,7 +18,7 @@
 // Bound: one K block of a 32 x 256 tile is 1,536 cycles of MFMA a SIMD.  In the
 // gate/up products of 2000 tokens (two workgroups a CU) the counters give 45% of
 // the time in MFMA, each of a SIMD's two waves 23% in vector work (E4M3 to bf16,
-// the split, the sums) and 18% waiting for memory or a barrier, and the LDS 30%
+// the split, the sums) and 20% waiting for memory or a barrier, and the LDS 30%
 // busy: vector work and MFMA hardly overlap.  Two f16 terms (hi + lo, 23 bits, and
 // fewer beside elements 2^16 times larger) took 555 us where the layer takes 630;
 // the error against 64 bits is 2.2e-7 for 2.4e-7, and of the projections at 385
@@ -383,8 +383,8 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void k_gemm_f32x(GemvMulti G, cons
 // subtiles are the gate and up rows of the same 32 outputs, h = silu(g) u as
 // f32; DOWN: 64 adjacent rows.  The shared expert's items (PS) run first in the
 // same launch; items and their XCD ranges as in k_gg.  2000 tokens of a
-// Qwen3-30B-A3B layer, Zipf(1.1): gate/up 425 us, down 230 us (medians of the
-// kernel trace).
+// Qwen3-30B-A3B layer, Zipf(1.1): gate/up 434 us, down 250 us (medians of the
+// kernel trace; least 366 and 209).
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void k_gg_f32x(GroupArgs G, GGProblem PR, GGProblem PS, const float *__restrict__ aR,
                                                     const float *__restrict__ aS) {

@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void k_route_tokens(GroupArgs G) {
 // workgroup of 1024 threads (16 waves) over the S*K slot ids (E <= CZ_MAX_E).
 // Up to CZ_DISPATCH_MAX slots a thread holds its slots' experts and ranks in
 // registers; above (WIDE) it passes over them in that many at a time, the ranks
-// waiting in slot_pos (16,000 slots: 17-23 us).  Each slot takes its rank among its
+// waiting in slot_pos (16,000 slots: 19-25 us).  Each slot takes its rank among its
 // expert's rows from an LDS atomic on the expert's count, the offsets come
 // from one prefix of the counts, and the slot goes to offset + rank.  Rows of
 // one expert come in the order the atomics were served, which is not fixed;

@@ -76,7 +76,11 @@ int colizig_cuda_matmul_fp8(float *y, const float *x, const unsigned char *w, co
  * colizig_hip_matmul_fp8_dev: y_dev[S,O] = x_dev[S,I] @ (e4m3(w) *
  * scales)^T with the matrix resident under key, asynchronous on `stream`
  * (NULL = the library's stream); x_dev, y_dev 16-byte aligned.  -7 key not
- * resident; -1 bad args or a shape other than the resident one; -4 launch. */
+ * resident; -1 bad args or a shape other than the resident one; -4 launch.
+ * A row's bits depend on the other rows of its call only through S: its sums
+ * are taken in one order up to 7 to 15 tokens (by I; the GEMV), in another to
+ * 128, to 512 and beyond, each at f32 accuracy.  The same holds for
+ * colizig_cuda_matmul_fp8. */
 int colizig_hip_matrix_load(uint64_t key, const unsigned char *w, const float *scales, int I, int O);
 int colizig_hip_matmul_fp8_dev(float *y_dev, const float *x_dev, int S, int I, int O, uint64_t key, void *stream);
 
@@ -286,7 +290,10 @@ uint64_t colizig_hip_set_scratch_limit(uint64_t bytes);
  * relative L2 bar either way: over a 48-layer Qwen3-30B-A3B prefill chain
  * (512 tokens, 64 checked against the oracle's own chain) the residual
  * stream is within 4.8e-5 (FP8) and 7.9e-7 (f16), and routing is bit-exact
- * at every layer in both modes.  FP8 runs about 2% faster. */
+ * at every layer in both modes.  FP8 runs about 2% faster.  The setting has no
+ * effect on calls of more than 8192 slots (S * topk): up to 65,536 their rows
+ * keep every f32 bit (2.2e-7 of a 64-bit layer at 2000 tokens), and longer
+ * calls run the per-token kernels. */
 int colizig_hip_set_prefill_fp8(int enable);
 int colizig_hip_fused_decode_active(uint32_t layer0, uint32_t nlayers, int S);
 int colizig_hip_chain_fused_times(uint32_t layer0, uint32_t nlayers, float *x_dev, float eps, int reps,

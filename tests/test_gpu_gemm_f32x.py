@@ -169,6 +169,27 @@ def test_small_elements_beside_large_ones(gpu, S, I):
 
 
 @pytest.mark.parametrize("S", [16, 129, 513])
+def test_rows_do_not_depend_on_each_other(gpu, S):
+    """Rows that take the large rows' path leave the bits of the others."""
+    rng = np.random.default_rng(S)
+    I, O = 384, 130
+    moe.set_vram_budget(1 << 30)
+    try:
+        w, s = synth.block_quantize(rng.normal(0, 0.02, size=(O, I)).astype(np.float32))
+        key = moe.Fp8Matrix.expert_key(74, S % 500, 1)
+        moe.matrix_load(key, w, s)
+        x = rng.normal(size=(S, I)).astype(np.float32)
+        y = _run(x, [(w, s, key)], I)[0]
+        odd = x.copy()
+        odd[1, 3], odd[4, 300], odd[9], odd[S - 1, 130] = np.inf, np.nan, 3e38, -2e33
+        z = _run(odd, [(w, s, key)], I)[0]
+        same = np.setdiff1d(np.arange(S), [1, 4, 9, S - 1])
+        assert np.array_equal(f32_bits(y[same]), f32_bits(z[same]))
+    finally:
+        moe.set_vram_budget(0)
+
+
+@pytest.mark.parametrize("S", [16, 129, 513])
 @pytest.mark.parametrize("I", [256, 384])
 def test_largest_floats(gpu, S, I):
     """Rows whose products with the weights' bytes pass the largest float
