@@ -435,8 +435,9 @@ int ensure_grouped(const colizig_dims &d, int S, hipStream_t st) {
     if (!grouped_ok(d, S) || (grouped_f32x(d, S) && use_grouped(d, S))) return 0;
     if (!grouped_f32x(d, S)) return ensure_work_grouped(d, S);
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    CZ_CHECK(hipStreamIsCapturing(st, &cs), -4);
-    if (cs == hipStreamCaptureStatusNone) (void)ensure_work_grouped(d, S);
+    const bool known = hipStreamIsCapturing(st, &cs) == hipSuccess;
+    if (!known) (void)hipGetLastError();  // the legacy stream while another one captures
+    if (known && cs == hipStreamCaptureStatusNone) (void)ensure_work_grouped(d, S);
     return 0;
 }
 
